@@ -25,103 +25,113 @@ struct Blue {
     const cf *tab;
 };
 
-template <int DIR>
-__device__ __forceinline__ cf blue_chirp(const Blue &b, int e)
+// elements of a line at the input positions of PM's forward first pass and
+// at the output positions of its inverse last pass (the same ones: both have
+// radix rf[0])
+template <class PM> using BlueIn = Elems<PM, -1, 0, true>;
+template <class PM> using BlueOut = Elems<PM, +1, PM::np - 1, true>;
+
+// chirp a_(t+o) of a thread's elements
+template <class PM, class El>
+__device__ __forceinline__ void blue_load_chirp(cf (&ch)[PM::E], const Blue &b, const El &el)
 {
-    const cf a = b.tab[e];
-    return DIR < 0 ? a : mkc(a.x, -a.y);
+    el.load([&](int s, int o, int d) { ch[s] = at32(b.tab + o, d); });
+}
+
+// v <- chirped line (conjugated chirp for the inverse), zero past its end
+template <class PM, int DIR, class El>
+__device__ __forceinline__ void blue_apply_chirp(cf (&v)[PM::E], const cf (&ch)[PM::E], const El &el)
+{
+    el.all([&](int s, int o) {
+        const cf z = cmul(v[s], DIR < 0 ? ch[s] : mkc(ch[s].x, -ch[s].y));
+        v[s] = el.inside(o) ? z : mkc(0.f, 0.f);
+    });
 }
 
 // circular convolution with the chirp: v holds the chirped, zero-padded
 // line at PM's forward first-pass input positions on entry and the result
-// at PM's inverse last-pass output positions on exit.  HP: load the chirp's
-// spectrum before the forward transform's exchanges, so its (L2) latency
-// overlaps them (faster for the row kernels; the column kernels, with more
-// registers live, were slower with it)
-template <class PM, int DIR, bool HP, class Lds>
+// at PM's inverse last-pass output positions on exit.  The chirp's spectrum
+// is loaded before the last exchange of the forward transform; `hook` runs
+// before the last exchange of the inverse one.
+template <class PM, int DIR, class Lds, class Hook>
 __device__ __forceinline__ void blue_conv(cf (&v)[PM::E], const cf *tw, int t, const Lds &L,
-                                          const Blue &b)
+                                          const Blue &b, Hook &hook)
 {
     const cf *h = b.tab + b.n + (DIR < 0 ? 0 : PM::n);
-    if constexpr (HP) {
-        cf hv[PM::E];
-        for_outputs<PM, -1, PM::np - 1>(t, [&](int s, int e) { hv[s] = h[e]; });
-        compute<PM, -1, 0>(v, tw, t);
-        passes_from<PM, -1, 1>(v, tw, t, L);
-        for_outputs<PM, -1, PM::np - 1>(t, [&](int s, int e) { v[s] = cmul(v[s], hv[s]); (void) e; });
-    } else {
-        compute<PM, -1, 0>(v, tw, t);
-        passes_from<PM, -1, 1>(v, tw, t, L);
-        for_outputs<PM, -1, PM::np - 1>(t, [&](int s, int e) { v[s] = cmul(v[s], h[e]); });
-    }
+    const Elems<PM, -1, PM::np - 1> mid{t, PM::n};
+    cf hv[PM::E];
+    auto load_h = [&] { mid.load([&](int s, int o, int d) { hv[s] = at32(h + o, d); }); };
+    compute<PM, -1, 0>(v, tw, t);
+    Slots<PM> sl;
+    passes_from<PM, -1, 1, false>(v, tw, t, L, sl, load_h);
+    mid.all([&](int s, int) { v[s] = cmul(v[s], hv[s]); });
     compute<PM, +1, 0>(v, tw, t);
-    passes_from<PM, +1, 1>(v, tw, t, L);
+    passes_from<PM, +1, 1, true>(v, tw, t, L, sl, hook);
 }
 
-// one length-n transform of direction DIR: src(e) / dst(e, x) for e < n
-template <class PM, int DIR, bool HP, class Lds, class Src, class Dst>
+// one length-n transform of direction DIR, callbacks as line_fft
+template <class PM, int DIR, class Lds, class Src, class Pre, class Dst>
 __device__ __forceinline__ void blue_fft(cf (&v)[PM::E], const cf *tw, int t, const Lds &L,
-                                         const Blue &b, Src &src, Dst &dst)
+                                         const Blue &b, Src &src, Pre &pre, Dst &dst)
 {
-    const int n = b.n;
-    auto in = [&](int e) { return e < n ? cmul(src(e), blue_chirp<DIR>(b, e)) : mkc(0.f, 0.f); };
-    gather_global<PM, -1, 0>(v, t, in);
-    blue_conv<PM, DIR, HP>(v, tw, t, L, b);
-    for_outputs<PM, +1, PM::np - 1>(t, [&](int s, int e) {
-        if (e < n) dst(e, cmul(v[s], blue_chirp<DIR>(b, e)));
-    });
+    const BlueIn<PM> in{t, b.n};
+    const BlueOut<PM> out{t, b.n};
+    cf ch[PM::E] = {};
+    src(v, in);
+    blue_load_chirp<PM>(ch, b, in);
+    blue_apply_chirp<PM, DIR>(v, ch, in);
+    auto hook = [&] {
+        blue_load_chirp<PM>(ch, b, out);
+        pre(out);
+    };
+    blue_conv<PM, DIR>(v, tw, t, L, b, hook);
+    blue_apply_chirp<PM, DIR>(v, ch, out);
+    dst(v, out);
 }
 
-// transform DA, mid(e, z, pre(e)) on its outputs, transform DB (as line_pair)
-template <class PM, int DA, int DB, bool HP, class Lds, class Src, class Pre, class Mid, class Dst>
+// transform DA, mid on its outputs, transform DB, callbacks as line_pair
+template <class PM, int DA, int DB, bool EARLY, class Lds, class Src, class Pre, class Mid, class Dst>
 __device__ __forceinline__ void blue_pair(cf (&v)[PM::E], const cf *tw, int t, const Lds &L,
                                           const Blue &b, Src &src, Pre &pre, Mid &mid, Dst &dst)
 {
     static_assert(DA == -DB, "a pair runs opposite directions");
-    const int n = b.n;
-    using PT = decltype(pre(0));
-    PT pf[PM::E];
-    auto in = [&](int e) { return e < n ? cmul(src(e), blue_chirp<DA>(b, e)) : mkc(0.f, 0.f); };
-    gather_global<PM, -1, 0>(v, t, in);
-    for_outputs<PM, +1, PM::np - 1>(t, [&](int s, int e) {
-        if (e < n) pf[s] = pre(e);
-    });
-    blue_conv<PM, DA, HP>(v, tw, t, L, b);
-    for_outputs<PM, +1, PM::np - 1>(t, [&](int s, int e) {
-        if (e < n) {
-            const cf z = mid(e, cmul(v[s], blue_chirp<DA>(b, e)), pf[s]);
-            v[s] = cmul(z, blue_chirp<DB>(b, e));
-        } else {
-            v[s] = mkc(0.f, 0.f);
-        }
-    });
-    blue_conv<PM, DB, HP>(v, tw, t, L, b);
-    for_outputs<PM, +1, PM::np - 1>(t, [&](int s, int e) {
-        if (e < n) dst(e, cmul(v[s], blue_chirp<DB>(b, e)));
-    });
+    const BlueIn<PM> in{t, b.n};
+    const BlueOut<PM> out{t, b.n};
+    cf ch[PM::E] = {};
+    src(v, in);
+    blue_load_chirp<PM>(ch, b, in);
+    if constexpr (EARLY) pre(out);
+    blue_apply_chirp<PM, DA>(v, ch, in);
+    auto at_mid = [&] {
+        blue_load_chirp<PM>(ch, b, out);
+        if constexpr (!EARLY) pre(out);
+    };
+    blue_conv<PM, DA>(v, tw, t, L, b, at_mid);
+    blue_apply_chirp<PM, DA>(v, ch, out);
+    mid(v, out);
+    blue_apply_chirp<PM, DB>(v, ch, out);
+    auto at_end = [&] { blue_load_chirp<PM>(ch, b, out); };
+    blue_conv<PM, DB>(v, tw, t, L, b, at_end);
+    blue_apply_chirp<PM, DB>(v, ch, out);
+    dst(v, out);
 }
-
-}  // namespace imr
-
-namespace imr {
 
 // direct (compiled plan of the line length) or Bluestein (BL: P is the
 // convolution plan, the line length is b.n) line transforms
-template <class P, int DIR, bool BL, bool HP = false, class Lds, class Src, class Dst>
+template <class P, int DIR, bool BL, class Lds, class Src, class Pre, class Dst>
 __device__ __forceinline__ void xfft(cf (&v)[P::E], const cf *tw, int t, const Lds &L, const Blue &b,
-                                     Src &src, Dst &dst)
+                                     Src &src, Pre &pre, Dst &dst)
 {
-    if constexpr (BL) blue_fft<P, DIR, HP>(v, tw, t, L, b, src, dst);
-    else line_fft<P, DIR>(v, tw, t, L, src, dst);
+    if constexpr (BL) blue_fft<P, DIR>(v, tw, t, L, b, src, pre, dst);
+    else line_fft<P, DIR>(v, tw, t, L, src, pre, dst);
 }
 
-template <class P, int DA, int DB, bool BL, bool HP = false, class Lds, class Src, class Pre, class Mid,
-          class Dst>
+template <class P, int DA, int DB, bool BL, bool EARLY, class Lds, class Src, class Pre, class Mid, class Dst>
 __device__ __forceinline__ void xpair(cf (&v)[P::E], const cf *tw, int t, const Lds &L, const Blue &b,
                                       Src &src, Pre &pre, Mid &mid, Dst &dst)
 {
-    if constexpr (BL) blue_pair<P, DA, DB, HP>(v, tw, t, L, b, src, pre, mid, dst);
-    else line_pair<P, DA, DB>(v, tw, t, L, src, pre, mid, dst);
+    if constexpr (BL) blue_pair<P, DA, DB, EARLY>(v, tw, t, L, b, src, pre, mid, dst);
+    else line_pair<P, DA, DB, EARLY>(v, tw, t, L, src, pre, mid, dst);
 }
 
 }  // namespace imr

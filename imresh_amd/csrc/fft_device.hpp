@@ -24,6 +24,15 @@
 
 #include "common.hpp"
 
+#ifndef IMR_WHEN
+#define IMR_WHEN 0
+#endif
+#ifndef IMR_WB
+#define IMR_WB 4
+#endif
+#ifndef IMR_WBL
+#define IMR_WBL 3
+#endif
 namespace imr {
 
 // native 2-wide vector: one 64-bit load / store per complex value
@@ -34,6 +43,21 @@ __device__ __forceinline__ cf mkc(float x, float y)
     r.x = x;
     r.y = y;
     return r;
+}
+
+// Global access at a workgroup-uniform base plus a 32-bit element index:
+// base + zext(idx * sizeof(T)) maps onto the scalar-base + 32-bit vector
+// offset addressing of global loads/stores (callers keep idx * sizeof(T)
+// below 4 GiB: at most 8192 x 8192 complex values).
+template <class T>
+__device__ __forceinline__ T &at32(T *base, unsigned idx)
+{
+    return *(T *) ((char *) base + (unsigned) (idx * (unsigned) sizeof(T)));
+}
+template <class T>
+__device__ __forceinline__ const T &at32(const T *base, unsigned idx)
+{
+    return *(const T *) ((const char *) base + (unsigned) (idx * (unsigned) sizeof(T)));
 }
 
 // ------------------------------------------------------------ complex math
@@ -228,39 +252,39 @@ __device__ __forceinline__ void bfly(cf *v)
 }
 
 // ------------------------------------------------------------ LDS layout
-// One padding slot every 32 values spreads the stride-R scatters of the
-// early passes over the LDS banks.
-__host__ __device__ constexpr int lpad(int i) { return i + (i >> 5); }
-__host__ __device__ constexpr int lds_elems(int n) { return n + (n >> 5) + 1; }
+// One padding slot every 16 values spreads the stride-R accesses of the
+// passes over the LDS banks (two 4-byte banks per complex value).
+__host__ __device__ constexpr int lpad(int i) { return i + (i >> 4); }
+__host__ __device__ constexpr int lds_elems(int n) { return n + (n >> 4) + 1; }
 
-// One line in LDS: element e at p[lpad(base + e*STRIDE)].  LdsC holds
-// complex values; LdsS holds one float component at a time (the exchange
-// then runs once for the real and once for the imaginary parts, halving the
-// LDS footprint of a tile).  at<STEP>(e0, r) addresses element e0 + r*STEP:
-// when STEP*STRIDE is a multiple of 32 the padded index is affine in r, so
-// the r-offsets become immediate offsets of the LDS instructions.
-template <int STEP, int STRIDE>
-__device__ __forceinline__ int lds_index(int base, int e0, int r)
-{
-    constexpr int d = STEP * STRIDE;
-    const int x0 = base + e0 * STRIDE;
-    if constexpr (d % 32 == 0) return lpad(x0) + r * (d / 32 * 33);
-    else return lpad(x0 + r * d);
-}
-
-template <int STRIDE>
-struct LdsC {
+// One line in LDS, slots of STRIDE lines interleaved: slot e at
+// p[lpad(e*STRIDE)].  at<STEP, MUL>(e0, r) addresses slot e0 + r*STEP for an
+// e0 that is a multiple of MUL: where the padding allows it, r moves the
+// address by a constant, which becomes an immediate offset of the LDS
+// instruction.  sync() orders a line's writes before its reads: a line whose
+// threads share one wave (WAVE) needs no workgroup barrier, for the LDS
+// executes a wave's instructions in order.
+template <int STRIDE, bool WAVE>
+struct LdsLine {
     cf *p;
-    int base;
-    template <int STEP>
-    __device__ __forceinline__ cf &at(int e0, int r) const { return p[lds_index<STEP, STRIDE>(base, e0, r)]; }
-};
-template <int STRIDE>
-struct LdsS {
-    float *p;
-    int base;
-    template <int STEP>
-    __device__ __forceinline__ float &at(int e0, int r) const { return p[lds_index<STEP, STRIDE>(base, e0, r)]; }
+    template <int STEP, int MUL>
+    __device__ __forceinline__ cf &at(int e0, int r) const
+    {
+        constexpr int d = STEP * STRIDE;
+        if constexpr (d % 16 == 0) return p[lpad(e0 * STRIDE) + r * (d / 16 * 17)];
+        else if constexpr ((MUL * STRIDE) % 16 == 0) return p[lpad(e0 * STRIDE) + lpad(r * d)];
+        else return p[lpad(e0 * STRIDE + r * d)];
+    }
+    __device__ __forceinline__ void sync() const
+    {
+        if constexpr (WAVE) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        } else {
+            __syncthreads();
+        }
+    }
 };
 
 // ------------------------------------------------------------ passes
@@ -274,20 +298,61 @@ struct PassOf {
     __device__ static constexpr bool full() { return nb % T == 0; }
 };
 
-// gather the inputs of pass I (natural positions j + r*nb) from global memory
-template <class P, int DIR, int I, class Src>
-__device__ __forceinline__ void gather_global(cf (&v)[P::E], int t, Src &src)
-{
+// The line elements a thread owns at pass I of direction DIR, where I reads
+// (a first pass) or writes (a last pass) the line in natural order: register
+// s holds element t + o with o = b*T + r*n/R known at compile time, so an
+// address is a uniform base moved by o (scalar registers) plus one per-lane
+// offset.  BL: the line is the first len <= n/2 of the plan's n elements.
+//
+// The callers load every operand of a step, then compute, then store: a
+// store between two loads orders them (the pointers may alias) and a wait
+// for the later load waits for the store too, a chain of one memory round
+// trip per element.
+template <class P, int DIR, int I, bool BL = false>
+struct Elems {
     using Q = PassOf<P, DIR, I>;
+    static_assert(I == 0 || I == P::np - 1, "natural order: the first or the last pass");
+    int t, len;
+
+    // f(s, o): every element of the plan
+    template <class F>
+    __device__ __forceinline__ void all(F &&f) const
+    {
 #pragma unroll
-    for (int b = 0; b < Q::B; ++b) {
-        const int j = t + b * Q::T;
-        if (Q::full() || j < Q::nb) {
+        for (int b = 0; b < Q::B; ++b) {
+            if (Q::full() || t + b * Q::T < Q::nb) {
 #pragma unroll
-            for (int r = 0; r < Q::R; ++r) v[b * Q::R + r] = src(j + r * Q::nb);
+                for (int r = 0; r < Q::R; ++r) f(b * Q::R + r, b * Q::T + r * Q::nb);
+            }
         }
     }
-}
+    // f(s, o, d): operand loads from o + d, where d = t except for the lanes
+    // past the end of a BL line, which repeat its last element
+    template <class F>
+    __device__ __forceinline__ void load(F &&f) const
+    {
+        all([&](int s, int o) {
+            if constexpr (BL) {
+                if (o < P::n / 2 && o < len) f(s, o, min(t, len - 1 - o));
+            } else {
+                f(s, o, t);
+            }
+        });
+    }
+    // f(s, o, d): the elements of the line, for stores
+    template <class F>
+    __device__ __forceinline__ void store(F &&f) const
+    {
+        all([&](int s, int o) {
+            if constexpr (BL) {
+                if (o < P::n / 2 && t + o < len) f(s, o, t);
+            } else {
+                f(s, o, t);
+            }
+        });
+    }
+    __device__ __forceinline__ bool inside(int o) const { return !BL || (o < P::n / 2 && t + o < len); }
+};
 
 // twiddles of pass I for this thread's butterflies (none for a first pass)
 template <class P, int DIR, int I>
@@ -343,164 +408,157 @@ __device__ __forceinline__ void compute(cf (&v)[P::E], const cf *__restrict__ tw
     compute_tw<P, DIR, I>(v, w, t);
 }
 
-// output positions of pass I: (j - j%ns)*R + j%ns + r*ns
-template <class P, int DIR, int I, class F>
-__device__ __forceinline__ void for_outputs(int t, F &&f)
+// Slots of the exchanges.  Pass I writes its outputs where it read its
+// inputs (register r of butterfly j to the slot of input r), so a slot
+// belongs to one thread from its read to its next write and an exchange needs
+// one barrier, between its writes and its reads, where a fixed slot per
+// element needs a second one before the writes.  (Measured with two barriers
+// and with one: see line_pair.)  slot<DIR, I, SECOND>(e) is the slot of
+// element e (of the Stockham order: the output positions of pass I-1, the
+// input positions of pass I) in the exchange before pass I:
+//   I = 1         e itself for the first transform of a chain; the second
+//                 transform of a pair (SECOND) starts in the slots that the
+//                 last pass of the first one read;
+//   I > 1         the slot of the input of pass I-1 that e replaced.
+// The radices of the two transforms of a pair are mirrored, so the pair's
+// last pass reads the slots its first pass wrote, and the next pair of a
+// chain starts over with slot = element.  slot is linear in r along a pass's
+// inputs e = j + r*n/R.
+template <class P, int DIR, int I, bool SECOND>
+__host__ __device__ constexpr unsigned slot(unsigned e)
+{
+    constexpr bool INV = DIR > 0;
+    if constexpr (I == 1) {
+        if constexpr (SECOND) {
+            constexpr unsigned R = P::rad(INV, 0);
+            return slot<P, -DIR, P::np - 1, false>(e / R + (e % R) * (P::n / R));
+        } else {
+            return e;
+        }
+    } else {
+        constexpr unsigned R = P::rad(INV, I - 1), NS = P::ns(INV, I - 1);
+        return slot<P, DIR, I - 1, SECOND>(e / (NS * R) * NS + e % NS + (e / NS) % R * (P::n / R));
+    }
+}
+
+// slot of input 0 of the thread's butterflies in the latest exchange
+template <class P> struct Slots {
+    int s[P::E];
+};
+
+// inputs of pass I from their slots
+template <class P, int DIR, int I, bool SECOND, class Lds>
+__device__ __forceinline__ void read_slots(cf (&v)[P::E], int t, const Lds &L, Slots<P> &at)
+{
+    using Q = PassOf<P, DIR, I>;
+    constexpr int STEP = (int) (slot<P, DIR, I, SECOND>(Q::nb) - slot<P, DIR, I, SECOND>(0));
+#pragma unroll
+    for (int b = 0; b < Q::B; ++b) {
+        const int j = t + b * Q::T;
+        if (Q::full() || j < Q::nb) {
+            at.s[b] = (int) slot<P, DIR, I, SECOND>((unsigned) j);
+#pragma unroll
+            for (int r = 0; r < Q::R; ++r) v[b * Q::R + r] = L.template at<STEP, 1>(at.s[b], r);
+        }
+    }
+}
+
+// outputs of pass I to the slots its inputs came from, which pass IR of
+// direction DR read (the pass itself, or the last pass of the transform
+// before it); a chain's first pass has read none and writes slot = element
+template <class P, int DIR, int I, int DR, int IR, bool SR, class Lds>
+__device__ __forceinline__ void write_slots(const cf (&v)[P::E], int t, const Lds &L, const Slots<P> &at)
 {
     using Q = PassOf<P, DIR, I>;
 #pragma unroll
     for (int b = 0; b < Q::B; ++b) {
         const int j = t + b * Q::T;
         if (Q::full() || j < Q::nb) {
-            const int k = j % Q::NS;
-            const int base = (j - k) * Q::R + k;
 #pragma unroll
-            for (int r = 0; r < Q::R; ++r) f(b * Q::R + r, base + r * Q::NS);
-        }
-    }
-}
-
-// input positions of pass I: j + r*nb
-template <class P, int DIR, int I, class F>
-__device__ __forceinline__ void for_inputs(int t, F &&f)
-{
-    using Q = PassOf<P, DIR, I>;
-#pragma unroll
-    for (int b = 0; b < Q::B; ++b) {
-        const int j = t + b * Q::T;
-        if (Q::full() || j < Q::nb) {
-#pragma unroll
-            for (int r = 0; r < Q::R; ++r) f(b * Q::R + r, j + r * Q::nb);
-        }
-    }
-}
-
-// scatter the outputs of the last pass to global memory (natural order)
-template <class P, int DIR, int I, class Dst>
-__device__ __forceinline__ void scatter_global(cf (&v)[P::E], int t, Dst &dst)
-{
-    for_outputs<P, DIR, I>(t, [&](int s, int e) { dst(e, v[s]); });
-}
-
-// elementwise operator on the natural-order outputs of a last pass
-template <class P, int DIR, int I, class Mid>
-__device__ __forceinline__ void apply_mid(cf (&v)[P::E], int t, Mid &mid)
-{
-    for_outputs<P, DIR, I>(t, [&](int s, int e) { v[s] = mid(e, v[s]); });
-}
-
-// LDS exchange between pass IA of direction DA (its outputs) and pass IB of
-// direction DB (its inputs): barrier, write, barrier, read.  The leading
-// barrier orders these writes after every read of the previous exchange, so
-// a wave that has read its inputs goes on to compute without waiting for
-// the others.  COMP selects the component moved (0 both as one complex,
-// 1 real part, 2 imaginary).
-template <class P, int DA, int IA, int DB, int IB, int COMP, class Lds>
-__device__ __forceinline__ void exchange_part(cf (&v)[P::E], int t, const Lds &L)
-{
-    using A = PassOf<P, DA, IA>;
-    using Bq = PassOf<P, DB, IB>;
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < A::B; ++b) {
-        const int j = t + b * A::T;
-        if (A::full() || j < A::nb) {
-            const int k = j % A::NS;
-            const int base = (j - k) * A::R + k;
-#pragma unroll
-            for (int r = 0; r < A::R; ++r) {
-                if constexpr (COMP == 0) L.template at<A::NS>(base, r) = v[b * A::R + r];
-                else if constexpr (COMP == 1) L.template at<A::NS>(base, r) = v[b * A::R + r].x;
-                else L.template at<A::NS>(base, r) = v[b * A::R + r].y;
-            }
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < Bq::B; ++b) {
-        const int j = t + b * Bq::T;
-        if (Bq::full() || j < Bq::nb) {
-#pragma unroll
-            for (int r = 0; r < Bq::R; ++r) {
-                if constexpr (COMP == 0) v[b * Bq::R + r] = L.template at<Bq::nb>(j, r);
-                else if constexpr (COMP == 1) v[b * Bq::R + r].x = L.template at<Bq::nb>(j, r);
-                else v[b * Bq::R + r].y = L.template at<Bq::nb>(j, r);
+            for (int r = 0; r < Q::R; ++r) {
+                if constexpr (IR == 0) {
+                    L.template at<1, Q::R>(j * Q::R, r) = v[b * Q::R + r];
+                } else {
+                    constexpr int STEP = (int) (slot<P, DR, IR, SR>(Q::nb) - slot<P, DR, IR, SR>(0));
+                    L.template at<STEP, 1>(at.s[b], r) = v[b * Q::R + r];
+                }
             }
         }
     }
 }
 
-template <class P, int DA, int IA, int DB, int IB, int S>
-__device__ __forceinline__ void exchange(cf (&v)[P::E], int t, const LdsC<S> &L)
+// passes [I, np) of direction DIR, each preceded by an LDS exchange; SECOND:
+// the transform follows one of the other direction in the same registers.
+// `hook` runs around the last exchange (WHEN): before it, so that loads
+// issued there are in flight during the exchange and the pass, or after the
+// last pass, which leaves the pass their registers.
+template <class P, int DIR, int I, bool SECOND, class Lds, class Hook>
+__device__ __forceinline__ void passes_from(cf (&v)[P::E], const cf *tw, int t, const Lds &L, Slots<P> &at,
+                                            Hook &hook)
 {
-    exchange_part<P, DA, IA, DB, IB, 0>(v, t, L);
-}
-template <class P, int DA, int IA, int DB, int IB, int S>
-__device__ __forceinline__ void exchange(cf (&v)[P::E], int t, const LdsS<S> &L)
-{
-    exchange_part<P, DA, IA, DB, IB, 1>(v, t, L);
-    exchange_part<P, DA, IA, DB, IB, 2>(v, t, L);
-}
-
-// passes [I, np) of direction DIR, each preceded by an LDS exchange
-template <class P, int DIR, int I, class Lds>
-__device__ __forceinline__ void passes_from(cf (&v)[P::E], const cf *tw, int t, const Lds &L)
-{
+    if constexpr (I == P::np && (P::np == 1 || IMR_WHEN == 0)) hook();
     if constexpr (I < P::np) {
         TwRegs<P, DIR, I> w;
         load_tw<P, DIR, I>(w, tw, t);
-        exchange<P, DIR, I - 1, DIR, I>(v, t, L);
+        if constexpr (I == P::np - 1 && IMR_WHEN == 2) hook();
+        if constexpr (I > 1) write_slots<P, DIR, I - 1, DIR, I - 1, SECOND>(v, t, L, at);
+        else if constexpr (SECOND) write_slots<P, DIR, 0, -DIR, P::np - 1, false>(v, t, L, at);
+        else write_slots<P, DIR, 0, DIR, 0, false>(v, t, L, at);
+        L.sync();
+        read_slots<P, DIR, I, SECOND>(v, t, L, at);
         compute_tw<P, DIR, I>(v, w, t);
-        passes_from<P, DIR, I + 1>(v, tw, t, L);
+        passes_from<P, DIR, I + 1, SECOND>(v, tw, t, L, at, hook);
     }
 }
 
-// One full transform: global (src) -> registers/LDS -> global (dst).
-template <class P, int DIR, class Lds, class Src, class Dst>
+struct NoHook {
+    __device__ __forceinline__ void operator()() const {}
+};
+
+// One full transform: src(v, in) fills the registers of the first pass,
+// dst(v, out) stores those of the last; pre(out) loads operands of dst.
+template <class P, int DIR, class Lds, class Src, class Pre, class Dst>
 __device__ __forceinline__ void line_fft(cf (&v)[P::E], const cf *tw, int t, const Lds &L, Src &src,
-                                         Dst &dst)
+                                         Pre &pre, Dst &dst)
 {
-    gather_global<P, DIR, 0>(v, t, src);
+    const Elems<P, DIR, 0> in{t, P::n};
+    const Elems<P, DIR, P::np - 1> out{t, P::n};
+    auto hook = [&] { pre(out); };
+    src(v, in);
     compute<P, DIR, 0>(v, tw, t);
-    passes_from<P, DIR, 1>(v, tw, t, L);
-    scatter_global<P, DIR, P::np - 1>(v, t, dst);
+    Slots<P> sl;
+    passes_from<P, DIR, 1, false>(v, tw, t, L, sl, hook);
+    dst(v, out);
 }
 
 // Transform in direction DA, elementwise `mid` on its natural-order output,
 // then the transform in direction DB.  A's last pass and B's first pass
 // have the same radix (mirrored sequences), so the junction never leaves
 // registers: B's first pass consumes exactly the positions A's last pass
-// produced in the same thread.  `pre(e)` runs right after the input gather,
-// so operands of `mid` read from global memory (pre returns them; `mid(e, z,
-// p)` receives them) are in flight during the first transform instead of
-// stalling the junction; a `pre` returning NoPre leaves the loads to `mid`.
-struct NoPre {};
-
-// the pair after its input gather: v holds the gathered line, pf the
-// prefetched junction operands
-template <class P, int DA, int DB, class Lds, class PT, class Mid, class Dst>
-__device__ __forceinline__ void line_pair_loaded(cf (&v)[P::E], PT (&pf)[P::E], const cf *tw, int t,
-                                                 const Lds &L, Mid &mid, Dst &dst)
-{
-    compute<P, DA, 0>(v, tw, t);
-    passes_from<P, DA, 1>(v, tw, t, L);
-    for_outputs<P, DA, P::np - 1>(t, [&](int s, int e) { v[s] = mid(e, v[s], pf[s]); });
-    compute<P, DB, 0>(v, tw, t);
-    passes_from<P, DB, 1>(v, tw, t, L);
-    scatter_global<P, DB, P::np - 1>(v, t, dst);
-}
-
-template <class P, int DA, int DB, class Lds, class Src, class Pre, class Mid, class Dst>
+// produced in the same thread.  `pre(at)` loads the operands of `mid` from
+// global memory: right after the input gather (EARLY), in flight during the
+// whole first transform, or before its last exchange, which holds their
+// registers for one pass instead of all.
+template <class P, int DA, int DB, bool EARLY, class Lds, class Src, class Pre, class Mid, class Dst>
 __device__ __forceinline__ void line_pair(cf (&v)[P::E], const cf *tw, int t, const Lds &L, Src &src,
                                           Pre &pre, Mid &mid, Dst &dst)
 {
     static_assert(DA == -DB, "a pair runs opposite directions");
     static_assert(P::rad(DA > 0, P::np - 1) == P::rad(DB > 0, 0), "mirrored junction radix");
-    using PT = decltype(pre(0));
-    PT pf[P::E];
-    gather_global<P, DA, 0>(v, t, src);
-    for_outputs<P, DA, P::np - 1>(t, [&](int s, int e) { pf[s] = pre(e); });
-    line_pair_loaded<P, DA, DB>(v, pf, tw, t, L, mid, dst);
+    const Elems<P, DA, 0> in{t, P::n};
+    const Elems<P, DA, P::np - 1> at{t, P::n};
+    const Elems<P, DB, P::np - 1> out{t, P::n};
+    auto hook = [&] { if constexpr (!EARLY) pre(at); };
+    NoHook none;
+    src(v, in);
+    if constexpr (EARLY) pre(at);
+    compute<P, DA, 0>(v, tw, t);
+    Slots<P> sl;
+    passes_from<P, DA, 1, false>(v, tw, t, L, sl, hook);
+    mid(v, at);
+    compute<P, DB, 0>(v, tw, t);
+    passes_from<P, DB, 1, true>(v, tw, t, L, sl, none);
+    dst(v, out);
 }
 
 // ------------------------------------------------------------ reductions

@@ -16,8 +16,6 @@
 #include "ops_device.hpp"
 #include "plans.hpp"
 
-#include <type_traits>
-
 #ifndef IMR_GROUP
 #error "compile with -DIMR_GROUP=<plan group>"
 #endif
@@ -28,12 +26,11 @@ namespace {
 
 enum ColKernel { CK_FWD, CK_INV, CK_PROJ, CK_FWD_REAL, CK_INV_REAL };
 
-// C columns per workgroup; SPLIT: exchange real and imaginary parts through
-// LDS one after the other (half the LDS of a complex tile); PF (CK_PROJ
+// C columns per workgroup; PF (CK_PROJ
 // only): the measured modulus is read right after the column gather instead
 // of at the junction.
-template <class P, int C, bool SPLIT, int K, bool PF = false, bool BL = false, int STG = 0>
-__global__ void __launch_bounds__(C *P::T) k_col(ColArgs a)
+template <class P, int C, int K, bool PF = false, bool BL = false, int STG = 0>
+__global__ void __launch_bounds__(C *P::T, P::E > 16 ? (IMR_WB ? 2 : 0) : BL ? IMR_WBL : IMR_WB) k_col(ColArgs a)
 {
     // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs
     // (workgroup x + y * gridDim.x to XCD (x + y * gridDim.x) mod 8), each
@@ -69,69 +66,80 @@ __global__ void __launch_bounds__(C *P::T) k_col(ColArgs a)
     const int col = bid * C + c;
     const bool valid = col < a.W;
     const int W = a.W;
-    // workgroup base (uniform) + 32-bit per-lane offsets e*W + c; columns past
-    // the edge read column 0 of the tile and never store
+    // workgroup base (uniform) + 32-bit per-lane offsets; columns past the
+    // edge read column 0 of the tile and never store
     const size_t wb = (size_t) b * a.istride + (size_t) sb * a.sub_xstride + (size_t) bid * C;
     const size_t mb = (size_t) b * a.istride + (size_t) sb * a.sub_mstride + (size_t) bid * C;
     const int MP = a.mpitch > 0 ? a.mpitch : W;   // row pitch of M (CK_PROJ)
     const int co = valid ? c : 0;
-    using Lds = std::conditional_t<SPLIT, LdsS<C>, LdsC<C>>;
-    const Lds L{(decltype(Lds::p)) smem, c};
+    const LdsLine<C, false> L{smem + c};
     const cf *tw = (const cf *) a.tw;
     cf v[P::E];
     const Blue bl{BL ? a.len : P::n, (const cf *) a.bs};
+    // element o + d of this lane's column of a plane with rows `pitch` apart
+    auto at = [=](auto *p, int o, int d, int pitch) -> auto & {
+        return at32(p + (size_t) ((unsigned) o * (unsigned) pitch), (unsigned) (d * pitch + co));
+    };
+    auto none = [](const auto &) {};
 
     if constexpr (K == CK_FWD || K == CK_INV || K == CK_FWD_REAL || K == CK_INV_REAL) {
         constexpr bool real_in = K == CK_FWD_REAL || K == CK_INV_REAL;
         constexpr int DIR = (K == CK_FWD || K == CK_FWD_REAL) ? -1 : +1;
         cf *out = (cf *) a.out + wb;
-        auto sl = [=](int e, cf x) { if (valid) at32(out, e * W + co) = x; };
+        auto sl = [&](auto &x, const auto &el) {
+            if (valid) el.store([&](int s, int o, int d) { at(out, o, d, W) = x[s]; });
+        };
         if constexpr (real_in) {
             const float *M = a.M + wb;
-            auto g0 = [=](int e) { return mkc(at32(M, e * W + co), 0.f); };
-            xfft<P, DIR, BL>(v, tw, t, L, bl, g0, sl);
+            auto g0 = [&](auto &x, const auto &el) {
+                el.load([&](int s, int o, int d) { x[s] = mkc(at(M, o, d, W), 0.f); });
+            };
+            xfft<P, DIR, BL>(v, tw, t, L, bl, g0, none, sl);
         } else {
             const cf *in = (const cf *) a.in + wb;
-            auto g0 = [=](int e) { return at32(in, e * W + co); };
-            xfft<P, DIR, BL>(v, tw, t, L, bl, g0, sl);
+            auto g0 = [&](auto &x, const auto &el) {
+                el.load([&](int s, int o, int d) { x[s] = at(in, o, d, W); });
+            };
+            xfft<P, DIR, BL>(v, tw, t, L, bl, g0, none, sl);
         }
     } else if constexpr (K == CK_PROJ) {
         cf *X = (cf *) a.X + wb;
         const float *M = a.M + mb;
-        auto g0 = [=](int e) { return at32(X, e * W + co); };
-        auto pre = [=](int e) {
-            if constexpr (PF) return at32(M, e * MP + co);
-            else return NoPre{};
+        float m[P::E];
+        auto g0 = [&](auto &x, const auto &el) {
+            el.load([&](int s, int o, int d) { x[s] = at(X, o, d, W); });
         };
-        auto mid = [=](int e, cf z, auto m) {
-            if constexpr (PF) return modulus_project_fused(z, m);
-            else return modulus_project_fused(z, at32(M, e * MP + co));
+        auto pre = [&](const auto &el) {
+            el.load([&](int s, int o, int d) { m[s] = at(M, o, d, MP); });
         };
-        auto sl = [=](int e, cf x) { if (valid) at32(X, e * W + co) = x; };
-        xpair<P, -1, +1, BL>(v, tw, t, L, bl, g0, pre, mid, sl);
+        auto mid = [&](auto &x, const auto &el) { modulus_project_line<P::E>(x, m, el); };
+        auto sl = [&](auto &x, const auto &el) {
+            if (valid) el.store([&](int s, int o, int d) { at(X, o, d, W) = x[s]; });
+        };
+        xpair<P, -1, +1, BL, PF>(v, tw, t, L, bl, g0, pre, mid, sl);
     }
 }
 
 // LDS bytes of a C-column tile
-template <class P, int C, bool SPLIT>
-constexpr size_t col_lds() { return (SPLIT ? sizeof(float) : sizeof(cf)) * (size_t) lds_elems(C * P::n); }
+template <class P, int C>
+constexpr size_t col_lds() { return sizeof(cf) * (size_t) lds_elems(C * P::n); }
 
-template <class P, int C, bool SPLIT, bool PF = false, bool BL = false, int STG = 0>
+template <class P, int C, bool PF = false, bool BL = false, int STG = 0>
 int launch_variant(int mode, ColArgs a, hipStream_t s)
 {
     static_assert(C * P::T <= 1024, "column workgroup too large");
-    static_assert(col_lds<P, C, SPLIT>() <= kLdsBudget, "column tile exceeds the LDS budget");
+    static_assert(col_lds<P, C>() <= kLdsBudget, "column tile exceeds the LDS budget");
     const int images = a.batch > 1 ? a.batch : 1;
     const dim3 grid((a.W + C - 1) / C, images * (a.sub > 1 ? a.sub : 1)), block(C * P::T);
-    constexpr size_t lds = col_lds<P, C, SPLIT>();
+    constexpr size_t lds = col_lds<P, C>();
     if constexpr (lds > 64 * 1024) {
         static const hipError_t attr = [&] {
             hipError_t e = hipSuccess;
-            for (const void *f : {(const void *) k_col<P, C, SPLIT, CK_FWD, false, BL>,
-                                  (const void *) k_col<P, C, SPLIT, CK_INV, false, BL>,
-                                  (const void *) k_col<P, C, SPLIT, CK_FWD_REAL, false, BL>,
-                                  (const void *) k_col<P, C, SPLIT, CK_INV_REAL, false, BL>,
-                                  (const void *) k_col<P, C, SPLIT, CK_PROJ, PF, BL, STG>})
+            for (const void *f : {(const void *) k_col<P, C, CK_FWD, false, BL>,
+                                  (const void *) k_col<P, C, CK_INV, false, BL>,
+                                  (const void *) k_col<P, C, CK_FWD_REAL, false, BL>,
+                                  (const void *) k_col<P, C, CK_INV_REAL, false, BL>,
+                                  (const void *) k_col<P, C, CK_PROJ, PF, BL, STG>})
                 if (e == hipSuccess)
                     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
             return e;
@@ -140,20 +148,20 @@ int launch_variant(int mode, ColArgs a, hipStream_t s)
     }
     switch (mode) {
     case COL_FWD:
-        IMR_LAUNCH((k_col<P, C, SPLIT, CK_FWD, false, BL>), grid, block, lds, s, a);
+        IMR_LAUNCH((k_col<P, C, CK_FWD, false, BL>), grid, block, lds, s, a);
         break;
     case COL_REAL_FWD:
-        IMR_LAUNCH((k_col<P, C, SPLIT, CK_FWD_REAL, false, BL>), grid, block, lds, s, a);
+        IMR_LAUNCH((k_col<P, C, CK_FWD_REAL, false, BL>), grid, block, lds, s, a);
         break;
     case COL_INV:
-        IMR_LAUNCH((k_col<P, C, SPLIT, CK_INV, false, BL>), grid, block, lds, s, a);
+        IMR_LAUNCH((k_col<P, C, CK_INV, false, BL>), grid, block, lds, s, a);
         break;
     case COL_INIT:
         a.out = a.X;
-        IMR_LAUNCH((k_col<P, C, SPLIT, CK_INV_REAL, false, BL>), grid, block, lds, s, a);
+        IMR_LAUNCH((k_col<P, C, CK_INV_REAL, false, BL>), grid, block, lds, s, a);
         break;
     case COL_PROJ:
-        IMR_LAUNCH((k_col<P, C, SPLIT, CK_PROJ, PF, BL, STG>), grid, block, lds, s, a);
+        IMR_LAUNCH((k_col<P, C, CK_PROJ, PF, BL, STG>), grid, block, lds, s, a);
         break;
     default: return IMRESH_ERR_INVALID;
     }
@@ -184,8 +192,8 @@ constexpr int col_variant_count() { return 2 * col_shape_count<N, Rs...>(); }
 template <class P, int C, int STG = 0>
 int launch_pf(bool pf, int mode, ColArgs a, hipStream_t s)
 {
-    return pf ? launch_variant<P, C, false, true, false, STG>(mode, a, s)
-              : launch_variant<P, C, false, false, false, STG>(mode, a, s);
+    return pf ? launch_variant<P, C, true, false, STG>(mode, a, s)
+              : launch_variant<P, C, false, false, STG>(mode, a, s);
 }
 
 template <int N, int... Rs>
@@ -200,10 +208,10 @@ int launch_col_variant(int var, int mode, ColArgs a, hipStream_t s)
         // the workgroups, half the LDS), each plain or prefetching
         constexpr int C2 = P16::C >= 2 ? P16::C / 2 : 1;
         switch (var - kBlueVariant) {
-        case 0: return launch_variant<P16, P16::C, false, false, true>(mode, a, s);
-        case 1: return launch_variant<P16, C2, false, false, true>(mode, a, s);
-        case 2: return launch_variant<P16, P16::C, false, true, true>(mode, a, s);
-        case 3: return launch_variant<P16, C2, false, true, true>(mode, a, s);
+        case 0: return launch_variant<P16, P16::C, false, true>(mode, a, s);
+        case 1: return launch_variant<P16, C2, false, true>(mode, a, s);
+        case 2: return launch_variant<P16, P16::C, true, true>(mode, a, s);
+        case 3: return launch_variant<P16, C2, true, true>(mode, a, s);
         default: break;
         }
     }

@@ -36,7 +36,7 @@ enum RowKernel { RK_FWD, RK_INV, RK_INVOUT, RK_FIRST, RK_MID, RK_FWD_NORM };
 // kRow* outputs / cut-off, fixed at compile time (a uniform runtime flag
 // tested per element slows the memory phases measurably)
 template <class P, int NL, int K, bool PF = false, bool BL = false, int STG = 0, int FL = 0>
-__global__ void __launch_bounds__(NL *P::T) k_row(RowArgs a)
+__global__ void __launch_bounds__(NL *P::T, P::E > 16 ? (IMR_WB ? 2 : 0) : BL ? IMR_WBL : IMR_WB) k_row(RowArgs a)
 {
     // image b of a batch (grid.y): its planes start b * istride elements in,
     // its scalars at b * kScalStride / kFlagStride
@@ -54,30 +54,41 @@ __global__ void __launch_bounds__(NL *P::T) k_row(RowArgs a)
     const int l = threadIdx.x / T, t = threadIdx.x - l * T;
     const int row = blockIdx.x * NL + l;
     const bool valid = row < a.H;
-    // workgroup base (uniform) + 32-bit per-lane offsets; rows past the end
+    // workgroup base (uniform) + 32-bit per-lane offset; rows past the end
     // read row 0 of the workgroup and never store
     const size_t wb = (size_t) b * a.istride + (size_t) blockIdx.x * NL * n;
-    const int lo = valid ? l * n : 0;
-    const LdsC<1> L{smem, l * P::n};
+    const unsigned lr = valid ? l * n : 0;
+    const LdsLine<1, 64 % T == 0> L{smem + l * lds_elems(P::n)};
     const cf *tw = (const cf *) a.tw;
     cf v[P::E];
     cf *X = (cf *) a.X + wb;
-    auto ldX = [=](int e) { return at32(X, lo + e); };
-    auto stX = [=](int e, cf x) { if (valid) at32(X, lo + e) = x; };
+    auto ldX = [&](auto &x, const auto &el) {
+        el.load([&](int s, int o, int d) { x[s] = at32(X + o, lr + d); });
+    };
+    auto stX = [&](auto &x, const auto &el) {
+        if (valid) el.store([&](int s, int o, int d) { at32(X + o, lr + d) = x[s]; });
+    };
+    auto none = [](const auto &) {};
 
     if constexpr (K == RK_FWD || K == RK_INV || K == RK_FWD_NORM) {
         const cf *in = (const cf *) a.in + wb;
-        auto g0 = [=](int e) { return at32(in, lo + e); };
+        auto g0 = [&](auto &x, const auto &el) {
+            el.load([&](int s, int o, int d) { x[s] = at32(in + o, lr + d); });
+        };
         if constexpr (K == RK_FWD_NORM) {
             // the last half of the forward model |FFT2(x)|
             // (diffractionIntensity.cpp:72-77): only |z| leaves the registers
             float *Bn = a.Bn + wb;
-            auto sl = [=](int e, cf x) { if (valid) at32(Bn, lo + e) = cnorm(x); };
-            xfft<P, -1, BL, true>(v, tw, t, L, bl, g0, sl);
+            auto sl = [&](auto &x, const auto &el) {
+                if (valid) el.store([&](int s, int o, int d) { at32(Bn + o, lr + d) = cnorm(x[s]); });
+            };
+            xfft<P, -1, BL>(v, tw, t, L, bl, g0, none, sl);
         } else {
             cf *out = (cf *) a.out + wb;
-            auto sl = [=](int e, cf x) { if (valid) at32(out, lo + e) = x; };
-            xfft<P, K == RK_FWD ? -1 : +1, BL, true>(v, tw, t, L, bl, g0, sl);
+            auto sl = [&](auto &x, const auto &el) {
+                if (valid) el.store([&](int s, int o, int d) { at32(out + o, lr + d) = x[s]; });
+            };
+            xfft<P, K == RK_FWD ? -1 : +1, BL>(v, tw, t, L, bl, g0, none, sl);
         }
     } else if constexpr (K == RK_INVOUT) {
         __shared__ float red_f[NL * P::T];
@@ -88,20 +99,29 @@ __global__ void __launch_bounds__(NL *P::T) k_row(RowArgs a)
         const uint8_t *mask = a.mask + wb;
         float err = 0.f;
         unsigned cnt = 0;
-        auto sl = [&](int e, cf g) {
-            if (!valid) return;
-            at32(X, lo + e) = g;
-            if constexpr ((fl & kRowWriteG) != 0) at32(G, lo + e) = g;
-            if constexpr ((fl & (kRowWriteBn | kRowError)) != 0) {
-                const float nrm = cnorm(g);
-                if constexpr ((fl & kRowWriteBn) != 0) at32(Bn, lo + e) = nrm;
-                if ((fl & kRowError) && at32(mask, lo + e)) {
-                    err += nrm;
-                    cnt += 1;
-                }
-            }
+        uint8_t m[P::E];
+        auto pre = [&](const auto &el) {
+            if constexpr ((fl & kRowError) != 0)
+                el.load([&](int s, int o, int d) { m[s] = at32(mask + o, lr + d); });
         };
-        xfft<P, +1, BL, true>(v, tw, t, L, bl, ldX, sl);
+        auto sl = [&](auto &x, const auto &el) {
+            if (!valid) return;
+            el.store([&](int s, int o, int d) {
+                at32(X + o, lr + d) = x[s];
+                if constexpr ((fl & kRowWriteG) != 0) at32(G + o, lr + d) = x[s];
+                if constexpr ((fl & (kRowWriteBn | kRowError)) != 0) {
+                    const float nrm = cnorm(x[s]);
+                    if constexpr ((fl & kRowWriteBn) != 0) at32(Bn + o, lr + d) = nrm;
+                    if constexpr ((fl & kRowError) != 0) {
+                        if (m[s]) {
+                            err += nrm;
+                            cnt += 1;
+                        }
+                    }
+                }
+            });
+        };
+        xfft<P, +1, BL>(v, tw, t, L, bl, ldX, pre, sl);
         if constexpr ((fl & kRowError) != 0) {
             err = block_reduce(err, red_f, [](float x, float y) { return x + y; });
             cnt = block_reduce(cnt, red_u, [](unsigned x, unsigned y) { return x + y; });
@@ -117,40 +137,44 @@ __global__ void __launch_bounds__(NL *P::T) k_row(RowArgs a)
         uint8_t *mask = a.mask + wb;
         const float *B2 = a.B2 + wb;
         const float beta = a.beta;
-        auto g0 = [=](int e) {
-            const cf g = at32(X, lo + e);
-            bool m;
-            if constexpr (cut) {
-                m = at32(B2, lo + e) < thr;
-                if (valid) at32(mask, lo + e) = m ? 1 : 0;
-            } else {
-                m = at32(mask, lo + e) == 1;
-            }
-            const cf gp = hio_constraint(at32(G, lo + e), g, m, beta);
-            if (valid) at32(G, lo + e) = gp;
-            return gp;
+        auto g0 = [&](auto &x, const auto &el) {
+            cf g[P::E];
+            float bv[P::E];
+            uint8_t m[P::E];
+            el.load([&](int s, int o, int d) {
+                x[s] = at32(X + o, lr + d);
+                g[s] = at32(G + o, lr + d);
+                if constexpr (cut) bv[s] = at32(B2 + o, lr + d);
+                else m[s] = at32(mask + o, lr + d);
+            });
+            el.all([&](int s, int o) {
+                if constexpr (cut) m[s] = bv[s] < thr ? 1 : 0;
+                x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta);
+            });
+            if (valid)
+                el.store([&](int s, int o, int d) {
+                    if constexpr (cut) at32(mask + o, lr + d) = m[s];
+                    at32(G + o, lr + d) = x[s];
+                });
         };
-        xfft<P, -1, BL, true>(v, tw, t, L, bl, g0, stX);
+        xfft<P, -1, BL>(v, tw, t, L, bl, g0, none, stX);
     } else if constexpr (K == RK_MID) {
         cf *G = (cf *) a.G + wb;
         const uint8_t *mask = a.mask + wb;
         const float beta = a.beta;
-        struct GM {
-            cf g;
-            bool m;
+        cf g[P::E];
+        uint8_t m[P::E];
+        auto pre = [&](const auto &el) {
+            el.load([&](int s, int o, int d) {
+                g[s] = at32(G + o, lr + d);
+                m[s] = at32(mask + o, lr + d);
+            });
         };
-        auto pre = [=](int e) {
-            if constexpr (PF) return GM{at32(G, lo + e), at32(mask, lo + e) == 1};
-            else return NoPre{};
+        auto mid = [&](auto &x, const auto &el) {
+            el.all([&](int s, int o) { x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta); });
+            if (valid) el.store([&](int s, int o, int d) { at32(G + o, lr + d) = x[s]; });
         };
-        auto mid = [=](int e, cf g, auto p) {
-            cf gp;
-            if constexpr (PF) gp = hio_constraint(p.g, g, p.m, beta);
-            else gp = hio_constraint(at32(G, lo + e), g, at32(mask, lo + e) == 1, beta);
-            if (valid) at32(G, lo + e) = gp;
-            return gp;
-        };
-        xpair<P, +1, -1, BL, true>(v, tw, t, L, bl, ldX, pre, mid, stX);
+        xpair<P, +1, -1, BL, PF>(v, tw, t, L, bl, ldX, pre, mid, stX);
     }
 }
 
@@ -159,12 +183,16 @@ constexpr int kInit = kRowWriteG | kRowWriteBn;
 constexpr int kLast = kRowWriteBn | kRowError;
 constexpr int kInitErr = kRowWriteG | kRowWriteBn | kRowError;
 
+// LDS bytes of an NL-row group
+template <int NL>
+constexpr size_t row_lds(int n) { return sizeof(cf) * (size_t) NL * lds_elems(n); }
+
 template <class P, int NL, bool PF = false, bool BL = false, int STG = 0>
 int launch_variant(int mode, RowArgs a, hipStream_t s)
 {
     static_assert(NL * P::T <= 1024, "row workgroup too large");
     const dim3 grid((a.H + NL - 1) / NL, a.batch > 1 ? a.batch : 1), block(NL * P::T);
-    constexpr size_t lds = sizeof(cf) * (size_t) lds_elems(NL * P::n);
+    constexpr size_t lds = row_lds<NL>(P::n);
     static_assert(lds <= kLdsBudget, "row tile exceeds the LDS budget");
     if constexpr (lds > 64 * 1024) {
         static const hipError_t attr = [&] {
@@ -223,7 +251,7 @@ constexpr int long_row_shapes()
 {
     using P16 = PlanE<16, N, Rs...>;
     return (2 * P16::L * P16::T <= 1024 &&
-            sizeof(cf) * (size_t) lds_elems(2 * P16::L * N) <= kLdsBudget) ? 4 : 2;
+            row_lds<2 * P16::L>(N) <= kLdsBudget) ? 4 : 2;
 }
 
 template <int N, int... Rs>

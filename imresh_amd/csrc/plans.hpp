@@ -74,7 +74,7 @@ struct PlanE {
             C /= 2;
         return C;
     }
-    __host__ __device__ static constexpr int lds_elems_c(int m) { return m + (m >> 5) + 1; }
+    __host__ __device__ static constexpr int lds_elems_c(int m) { return m + (m >> 4) + 1; }
     static constexpr int C = calc_C();
     static_assert(L * T <= 1024, "row workgroup too large");
     static_assert(C * T <= 1024, "column workgroup too large");
