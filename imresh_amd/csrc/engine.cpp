@@ -375,7 +375,10 @@ namespace {
 // ---------------------------------------------------------------- autotuner
 // Picks, per device and image size, the fastest row-pass and column-pass
 // kernel variant (element budget / rows or columns per workgroup / LDS
-// exchange) by timing each on a synthetic resident state with HIP events.
+// exchange) by timing each on a synthetic resident state with HIP events, the
+// row and the column pass in turn as an iteration runs them: alone, a pass of
+// 4096^2 finds its planes in the Infinity Cache, which the other pass leaves
+// only in part (column pass 115 us alone, 162 us in turn).
 // Runs once per (device, W, H) and process; IMRESH_AUTOTUNE=0 keeps the
 // defaults, IMRESH_VARIANTS=r,c forces a choice.
 int time_variant(bool row, int var, Plan2D p, Workspace *w, hipStream_t s, float *ms)
@@ -403,7 +406,8 @@ int time_variant(bool row, int var, Plan2D p, Workspace *w, hipStream_t s, float
         st = launch_fill_state(w->X, w->G, w->mask, w->M, w->Bn, w->n, w->W, s);
         for (int r = 0; r <= reps && st == IMRESH_OK; ++r) {
             if (r == 1) st = IMR_HIP_STATUS(hipEventRecord(e0, s));   // first launch warms up
-            if (st == IMRESH_OK) st = row ? launch_row(ROW_MID, p, ra, s) : launch_col(col_mode, p, ca, s);
+            if (st == IMRESH_OK && (row || col_mode == COL_PROJ)) st = launch_row(ROW_MID, p, ra, s);
+            if (st == IMRESH_OK && (!row || col_mode == COL_PROJ)) st = launch_col(col_mode, p, ca, s);
         }
         if (st == IMRESH_OK) st = IMR_HIP_STATUS(hipEventRecord(e1, s));
         if (st == IMRESH_OK) st = IMR_HIP_STATUS(hipEventSynchronize(e1));

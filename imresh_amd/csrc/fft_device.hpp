@@ -24,19 +24,11 @@
 
 #include "common.hpp"
 
-#ifndef IMR_WHEN
-#define IMR_WHEN 0
-#endif
-#ifndef IMR_WB
-#define IMR_WB 4
-#endif
-#ifndef IMR_WBL
-#define IMR_WBL 3
-#endif
 namespace imr {
 
 // native 2-wide vector: one 64-bit load / store per complex value
 typedef float cf __attribute__((ext_vector_type(2)));
+typedef float cf2 __attribute__((ext_vector_type(4)));   // two of them
 __device__ __forceinline__ cf mkc(float x, float y)
 {
     cf r;
@@ -45,20 +37,42 @@ __device__ __forceinline__ cf mkc(float x, float y)
     return r;
 }
 
-// Global access at a workgroup-uniform base plus a 32-bit element index:
-// base + zext(idx * sizeof(T)) maps onto the scalar-base + 32-bit vector
-// offset addressing of global loads/stores (callers keep idx * sizeof(T)
-// below 4 GiB: at most 8192 x 8192 complex values).
-template <class T>
-__device__ __forceinline__ T &at32(T *base, unsigned idx)
-{
-    return *(T *) ((char *) base + (unsigned) (idx * (unsigned) sizeof(T)));
-}
-template <class T>
-__device__ __forceinline__ const T &at32(const T *base, unsigned idx)
-{
-    return *(const T *) ((const char *) base + (unsigned) (idx * (unsigned) sizeof(T)));
-}
+// A plane in global memory: a workgroup-uniform base and size, one 32-bit
+// per-lane byte offset v and a uniform byte offset s.
+//
+// Loads go through a buffer descriptor: a thread's elements differ by uniform
+// offsets, so they share one vector register of address (plain pointers cost a
+// 64-bit vector add and a register pair per element), and the hardware range
+// check stands in for edge tests: a load past the end returns 0, kOutside is
+// past every end.
+// Stores go through plain pointers, and the caller keeps them inside: the
+// address arithmetic spaces a thread's stores.  Buffer stores, issued back to
+// back, were slower wherever a tile is narrower than a cache line (columns
+// of 4096^2: 2-D transform pair 258 against 227 us, 8192^2: 2164 against
+// 1630 us) and no faster elsewhere.
+constexpr unsigned kOutside = 0x80000000u;
+
+struct Buf {
+    __amdgpu_buffer_rsrc_t r;
+    char *p;
+    __device__ __forceinline__ Buf(const void *base, size_t bytes)
+        : r(__builtin_amdgcn_make_buffer_rsrc((void *) base, 0, (unsigned) bytes, 0x00027000)), p((char *) base)
+    {
+    }
+    template <class T>
+    __device__ __forceinline__ T get(unsigned v, unsigned s) const
+    {
+        if constexpr (sizeof(T) == 16) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0));
+        else if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0));
+        else if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0));
+        else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b8(r, v, s, 0));
+    }
+    template <class T>
+    __device__ __forceinline__ void put(T x, unsigned v, unsigned s) const
+    {
+        *(T *) (p + s + (size_t) v) = x;
+    }
+};
 
 // ------------------------------------------------------------ complex math
 // Products use one fma per component; the FFT is the only place that
@@ -287,6 +301,10 @@ struct LdsLine {
     }
 };
 
+// Keeps the loads issued above it above it: left alone, the scheduler sinks
+// each load to its use to save registers, one memory round trip per element.
+__device__ __forceinline__ void issue_loads() { __builtin_amdgcn_sched_barrier(0); }
+
 // ------------------------------------------------------------ passes
 // Pass I of plan P in direction DIR (forward: plan order, inverse: reversed).
 template <class P, int DIR, int I>
@@ -300,21 +318,21 @@ struct PassOf {
 
 // The line elements a thread owns at pass I of direction DIR, where I reads
 // (a first pass) or writes (a last pass) the line in natural order: register
-// s holds element t + o with o = b*T + r*n/R known at compile time, so an
-// address is a uniform base moved by o (scalar registers) plus one per-lane
-// offset.  BL: the line is the first len <= n/2 of the plan's n elements.
+// s holds element t + o with o = b*T + r*n/R known at compile time.  BL: the
+// line is the first len <= n/2 of the plan's n elements.
 //
 // The callers load every operand of a step, then compute, then store: a
-// store between two loads orders them (the pointers may alias) and a wait
-// for the later load waits for the store too, a chain of one memory round
-// trip per element.
+// store between two loads orders them (the planes may alias) and a wait for
+// the later load waits for the store too, a chain of one memory round trip
+// per element.
 template <class P, int DIR, int I, bool BL = false>
 struct Elems {
     using Q = PassOf<P, DIR, I>;
     static_assert(I == 0 || I == P::np - 1, "natural order: the first or the last pass");
+    static constexpr int span = BL ? P::n / 2 : P::n;   // len <= span
     int t, len;
 
-    // f(s, o): every element of the plan
+    // f(s, o): every element below span
     template <class F>
     __device__ __forceinline__ void all(F &&f) const
     {
@@ -322,36 +340,29 @@ struct Elems {
         for (int b = 0; b < Q::B; ++b) {
             if (Q::full() || t + b * Q::T < Q::nb) {
 #pragma unroll
-                for (int r = 0; r < Q::R; ++r) f(b * Q::R + r, b * Q::T + r * Q::nb);
+                for (int r = 0; r < Q::R; ++r)
+                    if (b * Q::T + r * Q::nb < span) f(b * Q::R + r, b * Q::T + r * Q::nb);
             }
         }
     }
-    // f(s, o, d): operand loads from o + d, where d = t except for the lanes
-    // past the end of a BL line, which repeat its last element
+    // f(s, o): operand loads, without the elements that lie past the end of
+    // the line for every thread
     template <class F>
     __device__ __forceinline__ void load(F &&f) const
     {
         all([&](int s, int o) {
-            if constexpr (BL) {
-                if (o < P::n / 2 && o < len) f(s, o, min(t, len - 1 - o));
-            } else {
-                f(s, o, t);
-            }
+            if (!BL || o < len) f(s, o);
         });
     }
-    // f(s, o, d): the elements of the line, for stores
+    // f(s, o): the elements of the line, for stores
     template <class F>
     __device__ __forceinline__ void store(F &&f) const
     {
         all([&](int s, int o) {
-            if constexpr (BL) {
-                if (o < P::n / 2 && t + o < len) f(s, o, t);
-            } else {
-                f(s, o, t);
-            }
+            if (inside(o)) f(s, o);
         });
     }
-    __device__ __forceinline__ bool inside(int o) const { return !BL || (o < P::n / 2 && t + o < len); }
+    __device__ __forceinline__ bool inside(int o) const { return !BL || t + o < len; }
 };
 
 // twiddles of pass I for this thread's butterflies (none for a first pass)
@@ -365,7 +376,7 @@ struct TwRegs {
 // global (L1/L2-resident) twiddle loads of pass I; issued before the LDS
 // exchange that precedes the pass so their latency overlaps the barrier
 template <class P, int DIR, int I>
-__device__ __forceinline__ void load_tw(TwRegs<P, DIR, I> &w, const cf *__restrict__ tw, int t)
+__device__ __forceinline__ void load_tw(TwRegs<P, DIR, I> &w, const Buf &tw, int t)
 {
     using Q = PassOf<P, DIR, I>;
     if constexpr (Q::NS > 1) {
@@ -373,9 +384,15 @@ __device__ __forceinline__ void load_tw(TwRegs<P, DIR, I> &w, const cf *__restri
         for (int b = 0; b < Q::B; ++b) {
             const int j = t + b * Q::T;
             if (Q::full() || j < Q::nb) {
-                const cf *p = tw + Q::TWOFF + (j % Q::NS) * (Q::R - 1);
+                const unsigned k = (unsigned) (j % Q::NS) * (8u * (Q::R - 1));
 #pragma unroll
-                for (int r = 1; r < Q::R; ++r) w.w[b * (Q::R - 1) + r - 1] = p[r - 1];
+                for (int r = 1; r + 1 < Q::R; r += 2) {
+                    const cf2 x = tw.get<cf2>(k + 8u * (r - 1), 8u * Q::TWOFF);
+                    w.w[b * (Q::R - 1) + r - 1] = mkc(x.x, x.y);
+                    w.w[b * (Q::R - 1) + r] = mkc(x.z, x.w);
+                }
+                if constexpr ((Q::R & 1) == 0)
+                    w.w[b * (Q::R - 1) + Q::R - 2] = tw.get<cf>(k + 8u * (Q::R - 2), 8u * Q::TWOFF);
             }
         }
     }
@@ -401,7 +418,7 @@ __device__ __forceinline__ void compute_tw(cf (&v)[P::E], const TwRegs<P, DIR, I
 }
 
 template <class P, int DIR, int I>
-__device__ __forceinline__ void compute(cf (&v)[P::E], const cf *__restrict__ tw, int t)
+__device__ __forceinline__ void compute(cf (&v)[P::E], const Buf &tw, int t)
 {
     TwRegs<P, DIR, I> w;
     load_tw<P, DIR, I>(w, tw, t);
@@ -412,8 +429,8 @@ __device__ __forceinline__ void compute(cf (&v)[P::E], const cf *__restrict__ tw
 // inputs (register r of butterfly j to the slot of input r), so a slot
 // belongs to one thread from its read to its next write and an exchange needs
 // one barrier, between its writes and its reads, where a fixed slot per
-// element needs a second one before the writes.  (Measured with two barriers
-// and with one: see line_pair.)  slot<DIR, I, SECOND>(e) is the slot of
+// element needs a second one before the writes.  (2048^2 projection pass:
+// 24.0 us with two barriers, 19.9 us with one.)  slot<DIR, I, SECOND>(e) is the slot of
 // element e (of the Stockham order: the output positions of pass I-1, the
 // input positions of pass I) in the exchange before pass I:
 //   I = 1         e itself for the first transform of a chain; the second
@@ -489,25 +506,29 @@ __device__ __forceinline__ void write_slots(const cf (&v)[P::E], int t, const Ld
 
 // passes [I, np) of direction DIR, each preceded by an LDS exchange; SECOND:
 // the transform follows one of the other direction in the same registers.
-// `hook` runs around the last exchange (WHEN): before it, so that loads
-// issued there are in flight during the exchange and the pass, or after the
-// last pass, which leaves the pass their registers.
-template <class P, int DIR, int I, bool SECOND, class Lds, class Hook>
-__device__ __forceinline__ void passes_from(cf (&v)[P::E], const cf *tw, int t, const Lds &L, Slots<P> &at,
+// `hook` loads operands of the step that follows: after the last pass, which
+// leaves the pass the registers, or (AHEAD) before its exchange, so that they
+// are in flight during the exchange and the pass.
+template <class P, int DIR, int I, bool SECOND, bool AHEAD, class Lds, class Hook>
+__device__ __forceinline__ void passes_from(cf (&v)[P::E], const Buf &tw, int t, const Lds &L, Slots<P> &at,
                                             Hook &hook)
 {
-    if constexpr (I == P::np && (P::np == 1 || IMR_WHEN == 0)) hook();
+    if constexpr (I == P::np && (P::np == 1 || !AHEAD)) {
+        hook();
+        issue_loads();
+    }
     if constexpr (I < P::np) {
         TwRegs<P, DIR, I> w;
         load_tw<P, DIR, I>(w, tw, t);
-        if constexpr (I == P::np - 1 && IMR_WHEN == 2) hook();
+        if constexpr (I == P::np - 1 && AHEAD) hook();
+        issue_loads();
         if constexpr (I > 1) write_slots<P, DIR, I - 1, DIR, I - 1, SECOND>(v, t, L, at);
         else if constexpr (SECOND) write_slots<P, DIR, 0, -DIR, P::np - 1, false>(v, t, L, at);
         else write_slots<P, DIR, 0, DIR, 0, false>(v, t, L, at);
         L.sync();
         read_slots<P, DIR, I, SECOND>(v, t, L, at);
         compute_tw<P, DIR, I>(v, w, t);
-        passes_from<P, DIR, I + 1, SECOND>(v, tw, t, L, at, hook);
+        passes_from<P, DIR, I + 1, SECOND, AHEAD>(v, tw, t, L, at, hook);
     }
 }
 
@@ -518,16 +539,17 @@ struct NoHook {
 // One full transform: src(v, in) fills the registers of the first pass,
 // dst(v, out) stores those of the last; pre(out) loads operands of dst.
 template <class P, int DIR, class Lds, class Src, class Pre, class Dst>
-__device__ __forceinline__ void line_fft(cf (&v)[P::E], const cf *tw, int t, const Lds &L, Src &src,
+__device__ __forceinline__ void line_fft(cf (&v)[P::E], const Buf &tw, int t, const Lds &L, Src &src,
                                          Pre &pre, Dst &dst)
 {
     const Elems<P, DIR, 0> in{t, P::n};
     const Elems<P, DIR, P::np - 1> out{t, P::n};
     auto hook = [&] { pre(out); };
     src(v, in);
+    issue_loads();
     compute<P, DIR, 0>(v, tw, t);
     Slots<P> sl;
-    passes_from<P, DIR, 1, false>(v, tw, t, L, sl, hook);
+    passes_from<P, DIR, 1, false, false>(v, tw, t, L, sl, hook);
     dst(v, out);
 }
 
@@ -536,11 +558,14 @@ __device__ __forceinline__ void line_fft(cf (&v)[P::E], const cf *tw, int t, con
 // have the same radix (mirrored sequences), so the junction never leaves
 // registers: B's first pass consumes exactly the positions A's last pass
 // produced in the same thread.  `pre(at)` loads the operands of `mid` from
-// global memory: right after the input gather (EARLY), in flight during the
-// whole first transform, or before its last exchange, which holds their
-// registers for one pass instead of all.
-template <class P, int DA, int DB, bool EARLY, class Lds, class Src, class Pre, class Mid, class Dst>
-__device__ __forceinline__ void line_pair(cf (&v)[P::E], const cf *tw, int t, const Lds &L, Src &src,
+// global memory, WHEN (a variant the autotuner picks by size): at the
+// junction itself, which costs no registers during the transform; ahead of
+// the first transform's last exchange; or early, right after the input
+// gather, in flight during the whole first transform.
+enum { kAtJunction = 0, kAhead = 1, kEarly = 2 };
+
+template <class P, int DA, int DB, int WHEN, class Lds, class Src, class Pre, class Mid, class Dst>
+__device__ __forceinline__ void line_pair(cf (&v)[P::E], const Buf &tw, int t, const Lds &L, Src &src,
                                           Pre &pre, Mid &mid, Dst &dst)
 {
     static_assert(DA == -DB, "a pair runs opposite directions");
@@ -548,16 +573,17 @@ __device__ __forceinline__ void line_pair(cf (&v)[P::E], const cf *tw, int t, co
     const Elems<P, DA, 0> in{t, P::n};
     const Elems<P, DA, P::np - 1> at{t, P::n};
     const Elems<P, DB, P::np - 1> out{t, P::n};
-    auto hook = [&] { if constexpr (!EARLY) pre(at); };
+    auto hook = [&] { if constexpr (WHEN != kEarly) pre(at); };
     NoHook none;
     src(v, in);
-    if constexpr (EARLY) pre(at);
+    if constexpr (WHEN == kEarly) pre(at);
+    issue_loads();
     compute<P, DA, 0>(v, tw, t);
     Slots<P> sl;
-    passes_from<P, DA, 1, false>(v, tw, t, L, sl, hook);
+    passes_from<P, DA, 1, false, WHEN == kAhead>(v, tw, t, L, sl, hook);
     mid(v, at);
     compute<P, DB, 0>(v, tw, t);
-    passes_from<P, DB, 1, true>(v, tw, t, L, sl, none);
+    passes_from<P, DB, 1, true, false>(v, tw, t, L, sl, none);
     dst(v, out);
 }
 

@@ -140,17 +140,12 @@ struct LinePlan {
 // fused projection: their own tile holds only 2 columns (16-byte rows)
 constexpr int kFourStepMinLine = 8192;
 
-// variant index of the Bluestein kernels: kBlueVariant + {0: the plan's
-// column tile, 1: half as many columns per workgroup, 2 / 3: the same with
-// the prefetching junction}; rows use kBlueVariant + {0: the plan's rows
-// per workgroup, 1: prefetching, 2: half as many rows}.  Sizes without a
-// plan are not tuned one by one (a server meets hundreds of them):
-// half-width column tiles measured fastest on every Bluestein size tried
-// (300-2039: 1-1.4x), and half-height row groups spread a mid-size image
-// over more CUs (700: row pass 19.5 -> 17.6 us), so both are fixed choices.
+// variant index of the Bluestein kernels.  Sizes without a plan are not tuned
+// one by one (a server meets hundreds of them): half-width column tiles
+// measured fastest on every Bluestein size tried (300-2039: 1-1.4x), and
+// half-height row groups spread a mid-size image over more CUs (700: row pass
+// 19.5 -> 17.6 us), so both are fixed choices.
 constexpr int kBlueVariant = 1000;
-constexpr int kBlueColDefault = 1;
-constexpr int kBlueRowDefault = 2;
 // longest line length: lengths without a compiled plan up to it run the
 // Bluestein kernels of a power-of-two convolution length up to 2 kMaxLine;
 // plans longer than kMaxLine exist only as such convolution lengths

@@ -26,11 +26,11 @@ namespace {
 
 enum ColKernel { CK_FWD, CK_INV, CK_PROJ, CK_FWD_REAL, CK_INV_REAL };
 
-// C columns per workgroup; PF (CK_PROJ
-// only): the measured modulus is read right after the column gather instead
-// of at the junction.
-template <class P, int C, int K, bool PF = false, bool BL = false, int STG = 0>
-__global__ void __launch_bounds__(C *P::T, P::E > 16 ? (IMR_WB ? 2 : 0) : BL ? IMR_WBL : IMR_WB) k_col(ColArgs a)
+// C columns per workgroup; WHEN (CK_PROJ only): where the measured modulus
+// is read (line_pair); BL: Bluestein kernels of column length a.len with P
+// the convolution plan.
+template <class P, int C, int K, int WHEN = kAtJunction, bool BL = false>
+__global__ void __launch_bounds__(C *P::T, 4) k_col(ColArgs a)
 {
     // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs
     // (workgroup x + y * gridDim.x to XCD (x + y * gridDim.x) mod 8), each
@@ -53,70 +53,67 @@ __global__ void __launch_bounds__(C *P::T, P::E > 16 ? (IMR_WB ? 2 : 0) : BL ? I
     const int sub = a.sub > 1 ? a.sub : 1;
     const int b = by / sub, sb = by - b * sub;
     if (a.done != nullptr && a.done[b * kFlagStride]) return;
-    if constexpr (STG > 0) {
-        // phase offset: the second half of the grid shares CUs with the first
-        // half; starting it STG x ~3.4 us later lets the loads of one overlap
-        // the arithmetic of the other instead of every workgroup loading,
-        // computing and storing in lockstep
-        if (blockIdx.x >= (gridDim.x >> 1))
-            for (int i = 0; i < STG; ++i) __builtin_amdgcn_s_sleep(127);
-    }
     extern __shared__ cf smem[];
     const int c = threadIdx.x % C, t = threadIdx.x / C;
     const int col = bid * C + c;
     const bool valid = col < a.W;
     const int W = a.W;
-    // workgroup base (uniform) + 32-bit per-lane offsets; columns past the
-    // edge read column 0 of the tile and never store
+    const int n = BL ? a.len : P::n;
     const size_t wb = (size_t) b * a.istride + (size_t) sb * a.sub_xstride + (size_t) bid * C;
-    const size_t mb = (size_t) b * a.istride + (size_t) sb * a.sub_mstride + (size_t) bid * C;
-    const int MP = a.mpitch > 0 ? a.mpitch : W;   // row pitch of M (CK_PROJ)
-    const int co = valid ? c : 0;
+    // planes from the tile's first element to the block's last row; lanes of
+    // columns past the edge load past every end
+    const size_t left = (size_t) n * W - (size_t) bid * C;
+    const unsigned c0 = (unsigned) c, out_of = valid ? 0u : kOutside;
+    const unsigned x0 = ((unsigned) (t * W) + c0) * 8u | out_of;
     const LdsLine<C, false> L{smem + c};
-    const cf *tw = (const cf *) a.tw;
+    const Buf tw(a.tw, 8 * (size_t) (2 * P::n - 1));
+    const Blue bl{n, Buf(a.bs, 8 * (size_t) (P::n / 2 + 2 * P::n))};
     cf v[P::E];
-    const Blue bl{BL ? a.len : P::n, (const cf *) a.bs};
-    // element o + d of this lane's column of a plane with rows `pitch` apart
-    auto at = [=](auto *p, int o, int d, int pitch) -> auto & {
-        return at32(p + (size_t) ((unsigned) o * (unsigned) pitch), (unsigned) (d * pitch + co));
+    auto ld = [&](const Buf &p) {
+        return [&](auto &x, const auto &el) {
+            el.load([&](int s, int o) { x[s] = p.template get<cf>(x0, 8u * (unsigned) o * (unsigned) W); });
+        };
+    };
+    auto st = [&](const Buf &p) {
+        return [&](auto &x, const auto &el) {
+            if (valid) el.store([&](int s, int o) { p.put(x[s], x0, 8u * (unsigned) o * (unsigned) W); });
+        };
     };
     auto none = [](const auto &) {};
 
     if constexpr (K == CK_FWD || K == CK_INV || K == CK_FWD_REAL || K == CK_INV_REAL) {
         constexpr bool real_in = K == CK_FWD_REAL || K == CK_INV_REAL;
         constexpr int DIR = (K == CK_FWD || K == CK_FWD_REAL) ? -1 : +1;
-        cf *out = (cf *) a.out + wb;
-        auto sl = [&](auto &x, const auto &el) {
-            if (valid) el.store([&](int s, int o, int d) { at(out, o, d, W) = x[s]; });
-        };
+        const Buf out(a.out + wb, 8 * left);
+        auto sl = st(out);
         if constexpr (real_in) {
-            const float *M = a.M + wb;
+            const Buf M(a.M + wb, 4 * left);
+            const unsigned m0 = ((unsigned) (t * W) + c0) * 4u | out_of;
             auto g0 = [&](auto &x, const auto &el) {
-                el.load([&](int s, int o, int d) { x[s] = mkc(at(M, o, d, W), 0.f); });
+                el.load([&](int s, int o) {
+                    x[s] = mkc(M.get<float>(m0, 4u * (unsigned) o * (unsigned) W), 0.f);
+                });
             };
             xfft<P, DIR, BL>(v, tw, t, L, bl, g0, none, sl);
         } else {
-            const cf *in = (const cf *) a.in + wb;
-            auto g0 = [&](auto &x, const auto &el) {
-                el.load([&](int s, int o, int d) { x[s] = at(in, o, d, W); });
-            };
+            const Buf in(a.in + wb, 8 * left);
+            auto g0 = ld(in);
             xfft<P, DIR, BL>(v, tw, t, L, bl, g0, none, sl);
         }
     } else if constexpr (K == CK_PROJ) {
-        cf *X = (cf *) a.X + wb;
-        const float *M = a.M + mb;
+        const int MP = a.mpitch > 0 ? a.mpitch : W;   // row pitch of M
+        const size_t mb = (size_t) b * a.istride + (size_t) sb * a.sub_mstride + (size_t) bid * C;
+        const Buf X(a.X + wb, 8 * left);
+        const Buf M(a.M + mb, 4 * ((size_t) (n - 1) * MP + W - (size_t) bid * C));
+        const unsigned m0 = ((unsigned) (t * MP) + c0) * 4u | out_of;
         float m[P::E];
-        auto g0 = [&](auto &x, const auto &el) {
-            el.load([&](int s, int o, int d) { x[s] = at(X, o, d, W); });
-        };
+        auto g0 = ld(X);
         auto pre = [&](const auto &el) {
-            el.load([&](int s, int o, int d) { m[s] = at(M, o, d, MP); });
+            el.load([&](int s, int o) { m[s] = M.get<float>(m0, 4u * (unsigned) o * (unsigned) MP); });
         };
         auto mid = [&](auto &x, const auto &el) { modulus_project_line<P::E>(x, m, el); };
-        auto sl = [&](auto &x, const auto &el) {
-            if (valid) el.store([&](int s, int o, int d) { at(X, o, d, W) = x[s]; });
-        };
-        xpair<P, -1, +1, BL, PF>(v, tw, t, L, bl, g0, pre, mid, sl);
+        auto sl = st(X);
+        xpair<P, -1, +1, BL, WHEN>(v, tw, t, L, bl, g0, pre, mid, sl);
     }
 }
 
@@ -124,7 +121,7 @@ __global__ void __launch_bounds__(C *P::T, P::E > 16 ? (IMR_WB ? 2 : 0) : BL ? I
 template <class P, int C>
 constexpr size_t col_lds() { return sizeof(cf) * (size_t) lds_elems(C * P::n); }
 
-template <class P, int C, bool PF = false, bool BL = false, int STG = 0>
+template <class P, int C, int WHEN = kAtJunction, bool BL = false>
 int launch_variant(int mode, ColArgs a, hipStream_t s)
 {
     static_assert(C * P::T <= 1024, "column workgroup too large");
@@ -132,14 +129,15 @@ int launch_variant(int mode, ColArgs a, hipStream_t s)
     const int images = a.batch > 1 ? a.batch : 1;
     const dim3 grid((a.W + C - 1) / C, images * (a.sub > 1 ? a.sub : 1)), block(C * P::T);
     constexpr size_t lds = col_lds<P, C>();
+    constexpr int AJ = kAtJunction;
     if constexpr (lds > 64 * 1024) {
         static const hipError_t attr = [&] {
             hipError_t e = hipSuccess;
-            for (const void *f : {(const void *) k_col<P, C, CK_FWD, false, BL>,
-                                  (const void *) k_col<P, C, CK_INV, false, BL>,
-                                  (const void *) k_col<P, C, CK_FWD_REAL, false, BL>,
-                                  (const void *) k_col<P, C, CK_INV_REAL, false, BL>,
-                                  (const void *) k_col<P, C, CK_PROJ, PF, BL, STG>})
+            for (const void *f : {(const void *) k_col<P, C, CK_FWD, AJ, BL>,
+                                  (const void *) k_col<P, C, CK_INV, AJ, BL>,
+                                  (const void *) k_col<P, C, CK_FWD_REAL, AJ, BL>,
+                                  (const void *) k_col<P, C, CK_INV_REAL, AJ, BL>,
+                                  (const void *) k_col<P, C, CK_PROJ, WHEN, BL>})
                 if (e == hipSuccess)
                     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
             return e;
@@ -147,98 +145,61 @@ int launch_variant(int mode, ColArgs a, hipStream_t s)
         if (attr != hipSuccess) return from_hip(attr);
     }
     switch (mode) {
-    case COL_FWD:
-        IMR_LAUNCH((k_col<P, C, CK_FWD, false, BL>), grid, block, lds, s, a);
-        break;
-    case COL_REAL_FWD:
-        IMR_LAUNCH((k_col<P, C, CK_FWD_REAL, false, BL>), grid, block, lds, s, a);
-        break;
-    case COL_INV:
-        IMR_LAUNCH((k_col<P, C, CK_INV, false, BL>), grid, block, lds, s, a);
-        break;
+    case COL_FWD: IMR_LAUNCH((k_col<P, C, CK_FWD, AJ, BL>), grid, block, lds, s, a); break;
+    case COL_REAL_FWD: IMR_LAUNCH((k_col<P, C, CK_FWD_REAL, AJ, BL>), grid, block, lds, s, a); break;
+    case COL_INV: IMR_LAUNCH((k_col<P, C, CK_INV, AJ, BL>), grid, block, lds, s, a); break;
     case COL_INIT:
         a.out = a.X;
-        IMR_LAUNCH((k_col<P, C, CK_INV_REAL, false, BL>), grid, block, lds, s, a);
+        IMR_LAUNCH((k_col<P, C, CK_INV_REAL, AJ, BL>), grid, block, lds, s, a);
         break;
-    case COL_PROJ:
-        IMR_LAUNCH((k_col<P, C, CK_PROJ, PF, BL, STG>), grid, block, lds, s, a);
-        break;
+    case COL_PROJ: IMR_LAUNCH((k_col<P, C, CK_PROJ, WHEN, BL>), grid, block, lds, s, a); break;
     default: return IMRESH_ERR_INVALID;
     }
     return imr::launch_status(__FILE__, __LINE__);
 }
 
-// Column variants of a length (index: tile shape, then +count/2 for the
-// prefetching CK_PROJ): shape 0 = E 16 with the plan's default tile; for
-// long columns also 1 = E 32 (half the threads per column, 512-thread
-// groups), 2 = E 16 with 4-column tiles (two workgroups per CU) and 3, 4 =
-// the same with the second half of the grid started ~3.4 / ~6.8 us late.
-template <int N>
-constexpr bool blue_length() { return N >= 64 && N <= 2 * kMaxLine && (N & (N - 1)) == 0; }
-
+// Column variants of a length: index = when * shapes + shape.  `when` is where
+// CK_PROJ reads the modulus (line_pair); shape 0 has the plan's tile, shape 1
+// (1024 and 2048 points) 4-column tiles, twice the workgroups.
 template <int N, int... Rs>
 constexpr int col_shape_count()
 {
-    using P16 = PlanE<16, N, Rs...>;
-    constexpr bool pow2 = (N & (N - 1)) == 0;   // extra shapes for the power-of-two lengths
-    if constexpr (N >= 1024 && pow2 && P16::C > 4) return 5;
-    else if constexpr (N >= 1024 && pow2) return 2;
-    return 1;
+    return N >= 1024 && (N & (N - 1)) == 0 && Plan<N, Rs...>::C > 4 ? 2 : 1;
 }
 
 template <int N, int... Rs>
-constexpr int col_variant_count() { return 2 * col_shape_count<N, Rs...>(); }
+constexpr int col_variant_count() { return 3 * col_shape_count<N, Rs...>(); }
 
-template <class P, int C, int STG = 0>
-int launch_pf(bool pf, int mode, ColArgs a, hipStream_t s)
+// Bluestein kernels exist for the power-of-two convolution lengths, with half
+// as many columns per tile as the plan (measured fastest, see kBlueVariant)
+template <int N>
+constexpr bool blue_length() { return N >= 64 && N <= 2 * kMaxLine && (N & (N - 1)) == 0; }
+
+template <class P, int C>
+int launch_when(int when, int mode, ColArgs a, hipStream_t s)
 {
-    return pf ? launch_variant<P, C, true, false, STG>(mode, a, s)
-              : launch_variant<P, C, false, false, STG>(mode, a, s);
+    if (when == kEarly) return launch_variant<P, C, kEarly>(mode, a, s);
+    if (when == kAhead) return launch_variant<P, C, kAhead>(mode, a, s);
+    return launch_variant<P, C>(mode, a, s);
 }
-
-template <int N, int... Rs>
-int launch_col_direct(int var, int mode, ColArgs a, hipStream_t s);
 
 template <int N, int... Rs>
 int launch_col_variant(int var, int mode, ColArgs a, hipStream_t s)
 {
-    using P16 = PlanE<16, N, Rs...>;
+    using P = Plan<N, Rs...>;
     if constexpr (blue_length<N>()) {
-        // Bluestein variants: the plan's tile or half as many columns (twice
-        // the workgroups, half the LDS), each plain or prefetching
-        constexpr int C2 = P16::C >= 2 ? P16::C / 2 : 1;
-        switch (var - kBlueVariant) {
-        case 0: return launch_variant<P16, P16::C, false, true>(mode, a, s);
-        case 1: return launch_variant<P16, C2, false, true>(mode, a, s);
-        case 2: return launch_variant<P16, P16::C, true, true>(mode, a, s);
-        case 3: return launch_variant<P16, C2, true, true>(mode, a, s);
-        default: break;
-        }
+        if (var == kBlueVariant)
+            return launch_variant<P, (P::C >= 2 ? P::C / 2 : 1), kAtJunction, true>(mode, a, s);
     }
     if constexpr (N > kMaxLine) {
         return IMRESH_ERR_UNSUPPORTED_SIZE;   // a convolution length only
     } else {
-        return launch_col_direct<N, Rs...>(var, mode, a, s);
-    }
-}
-
-template <int N, int... Rs>
-int launch_col_direct(int var, int mode, ColArgs a, hipStream_t s)
-{
-    using P16 = PlanE<16, N, Rs...>;
-    constexpr int ns = col_shape_count<N, Rs...>();
-    const bool pf = var >= ns;
-    const int shape = pf ? var - ns : var;
-    if constexpr (ns > 1) {
-        using P32 = PlanE<32, N, Rs...>;
-        if (shape == 1) return launch_pf<P32, P32::C>(pf, mode, a, s);
-        if constexpr (ns == 5) {
-            if (shape == 2) return launch_pf<P16, 4>(pf, mode, a, s);
-            if (shape == 3) return launch_pf<P16, 4, 1>(pf, mode, a, s);
-            if (shape == 4) return launch_pf<P16, 4, 2>(pf, mode, a, s);
+        constexpr int ns = col_shape_count<N, Rs...>();
+        if constexpr (ns > 1) {
+            if (var % ns == 1) return launch_when<P, 4>(var / ns, mode, a, s);
         }
+        return launch_when<P, P::C>(var / ns, mode, a, s);
     }
-    return launch_pf<P16, P16::C>(pf, mode, a, s);
 }
 
 template <int G, int N, int... Rs>

@@ -30,88 +30,82 @@ namespace {
 
 enum RowKernel { RK_FWD, RK_INV, RK_INVOUT, RK_FIRST, RK_MID, RK_FWD_NORM };
 
-// NL rows per workgroup; PF (RK_MID only): gPrev and the mask are read right
-// after the row gather instead of at the junction; BL: Bluestein kernels of
-// row length a.len with P the convolution plan; FL (RK_INVOUT, RK_FIRST): the
-// kRow* outputs / cut-off, fixed at compile time (a uniform runtime flag
-// tested per element slows the memory phases measurably)
-template <class P, int NL, int K, bool PF = false, bool BL = false, int STG = 0, int FL = 0>
-__global__ void __launch_bounds__(NL *P::T, P::E > 16 ? (IMR_WB ? 2 : 0) : BL ? IMR_WBL : IMR_WB) k_row(RowArgs a)
+// NL rows per workgroup; WHEN (RK_MID only): where gPrev and the mask are
+// read (line_pair); BL: Bluestein kernels of row length a.len with P the
+// convolution plan; FL (RK_INVOUT, RK_FIRST): the kRow* outputs / cut-off,
+// fixed at compile time (a uniform runtime flag tested per element slows the
+// memory phases measurably).  At least 4 waves per SIMD: with fewer, 2048
+// rows of 2048 points no longer run as one generation of workgroups.
+template <class P, int NL, int K, int WHEN = kAtJunction, bool BL = false, int FL = 0>
+__global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
 {
     // image b of a batch (grid.y): its planes start b * istride elements in,
     // its scalars at b * kScalStride / kFlagStride
     const int b = blockIdx.y;
     if (a.done != nullptr && a.done[b * kFlagStride]) return;
-    if constexpr (STG > 0) {
-        // phase offset of the second half of the grid (see k_col)
-        if (blockIdx.x >= (gridDim.x >> 1))
-            for (int i = 0; i < STG; ++i) __builtin_amdgcn_s_sleep(127);
-    }
     extern __shared__ cf smem[];
     constexpr int T = P::T;
     const int n = BL ? a.len : P::n;
-    const Blue bl{n, (const cf *) a.bs};
     const int l = threadIdx.x / T, t = threadIdx.x - l * T;
-    const int row = blockIdx.x * NL + l;
-    const bool valid = row < a.H;
-    // workgroup base (uniform) + 32-bit per-lane offset; rows past the end
-    // read row 0 of the workgroup and never store
+    // planes from the workgroup's first row to the image's last: loads of the
+    // rows past the end return 0
     const size_t wb = (size_t) b * a.istride + (size_t) blockIdx.x * NL * n;
-    const unsigned lr = valid ? l * n : 0;
+    const size_t left = (size_t) (a.H - (int) blockIdx.x * NL) * n;
+    const unsigned e0 = (unsigned) (l * n + t);
+    const bool valid = (int) blockIdx.x * NL + l < a.H;
+    const Buf X(a.X + wb, 8 * left), G(a.G + wb, 8 * left), mask(a.mask + wb, left), Bn(a.Bn + wb, 4 * left);
+    const Blue bl{n, Buf(a.bs, 8 * (size_t) (P::n / 2 + 2 * P::n))};
+    const Buf tw(a.tw, 8 * (size_t) (2 * P::n - 1));
     const LdsLine<1, 64 % T == 0> L{smem + l * lds_elems(P::n)};
-    const cf *tw = (const cf *) a.tw;
     cf v[P::E];
-    cf *X = (cf *) a.X + wb;
-    auto ldX = [&](auto &x, const auto &el) {
-        el.load([&](int s, int o, int d) { x[s] = at32(X + o, lr + d); });
+    auto ld = [&](const Buf &p) {
+        return [&](auto &x, const auto &el) {
+            el.load([&](int s, int o) { x[s] = p.template get<cf>(8 * e0, 8 * o); });
+        };
     };
-    auto stX = [&](auto &x, const auto &el) {
-        if (valid) el.store([&](int s, int o, int d) { at32(X + o, lr + d) = x[s]; });
+    auto st = [&](const Buf &p) {
+        return [&](auto &x, const auto &el) {
+            if (valid) el.store([&](int s, int o) { p.put(x[s], 8 * e0, 8 * o); });
+        };
     };
     auto none = [](const auto &) {};
+    auto stX = st(X);
 
     if constexpr (K == RK_FWD || K == RK_INV || K == RK_FWD_NORM) {
-        const cf *in = (const cf *) a.in + wb;
-        auto g0 = [&](auto &x, const auto &el) {
-            el.load([&](int s, int o, int d) { x[s] = at32(in + o, lr + d); });
-        };
+        const Buf in(a.in + wb, 8 * left);
+        auto g0 = ld(in);
         if constexpr (K == RK_FWD_NORM) {
             // the last half of the forward model |FFT2(x)|
             // (diffractionIntensity.cpp:72-77): only |z| leaves the registers
-            float *Bn = a.Bn + wb;
             auto sl = [&](auto &x, const auto &el) {
-                if (valid) el.store([&](int s, int o, int d) { at32(Bn + o, lr + d) = cnorm(x[s]); });
+                if (valid) el.store([&](int s, int o) { Bn.put(cnorm(x[s]), 4 * e0, 4 * o); });
             };
             xfft<P, -1, BL>(v, tw, t, L, bl, g0, none, sl);
         } else {
-            cf *out = (cf *) a.out + wb;
-            auto sl = [&](auto &x, const auto &el) {
-                if (valid) el.store([&](int s, int o, int d) { at32(out + o, lr + d) = x[s]; });
-            };
+            const Buf out(a.out + wb, 8 * left);
+            auto sl = st(out);
             xfft<P, K == RK_FWD ? -1 : +1, BL>(v, tw, t, L, bl, g0, none, sl);
         }
     } else if constexpr (K == RK_INVOUT) {
         __shared__ float red_f[NL * P::T];
         __shared__ unsigned red_u[NL * P::T];
         constexpr int fl = FL;
-        cf *G = (cf *) a.G + wb;
-        float *Bn = a.Bn + wb;
-        const uint8_t *mask = a.mask + wb;
         float err = 0.f;
         unsigned cnt = 0;
         uint8_t m[P::E];
+        auto ldX = ld(X);
         auto pre = [&](const auto &el) {
             if constexpr ((fl & kRowError) != 0)
-                el.load([&](int s, int o, int d) { m[s] = at32(mask + o, lr + d); });
+                el.load([&](int s, int o) { m[s] = mask.get<uint8_t>(e0, o); });
         };
         auto sl = [&](auto &x, const auto &el) {
             if (!valid) return;
-            el.store([&](int s, int o, int d) {
-                at32(X + o, lr + d) = x[s];
-                if constexpr ((fl & kRowWriteG) != 0) at32(G + o, lr + d) = x[s];
+            el.store([&](int s, int o) {
+                X.put(x[s], 8 * e0, 8 * o);
+                if constexpr ((fl & kRowWriteG) != 0) G.put(x[s], 8 * e0, 8 * o);
                 if constexpr ((fl & (kRowWriteBn | kRowError)) != 0) {
                     const float nrm = cnorm(x[s]);
-                    if constexpr ((fl & kRowWriteBn) != 0) at32(Bn + o, lr + d) = nrm;
+                    if constexpr ((fl & kRowWriteBn) != 0) Bn.put(nrm, 4 * e0, 4 * o);
                     if constexpr ((fl & kRowError) != 0) {
                         if (m[s]) {
                             err += nrm;
@@ -133,48 +127,45 @@ __global__ void __launch_bounds__(NL *P::T, P::E > 16 ? (IMR_WB ? 2 : 0) : BL ? 
     } else if constexpr (K == RK_FIRST) {
         constexpr bool cut = (FL & kRowCut) != 0;
         const float thr = cut ? a.thr[b * kScalStride] : 0.f;
-        cf *G = (cf *) a.G + wb;
-        uint8_t *mask = a.mask + wb;
-        const float *B2 = a.B2 + wb;
+        const Buf B2(a.B2 + wb, 4 * left);
         const float beta = a.beta;
         auto g0 = [&](auto &x, const auto &el) {
             cf g[P::E];
             float bv[P::E];
             uint8_t m[P::E];
-            el.load([&](int s, int o, int d) {
-                x[s] = at32(X + o, lr + d);
-                g[s] = at32(G + o, lr + d);
-                if constexpr (cut) bv[s] = at32(B2 + o, lr + d);
-                else m[s] = at32(mask + o, lr + d);
+            el.load([&](int s, int o) {
+                x[s] = X.get<cf>(8 * e0, 8 * o);
+                g[s] = G.get<cf>(8 * e0, 8 * o);
+                if constexpr (cut) bv[s] = B2.get<float>(4 * e0, 4 * o);
+                else m[s] = mask.get<uint8_t>(e0, o);
             });
-            el.all([&](int s, int o) {
+            el.load([&](int s, int) {
                 if constexpr (cut) m[s] = bv[s] < thr ? 1 : 0;
                 x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta);
             });
-            if (valid)
-                el.store([&](int s, int o, int d) {
-                    if constexpr (cut) at32(mask + o, lr + d) = m[s];
-                    at32(G + o, lr + d) = x[s];
-                });
+            if (!valid) return;
+            el.store([&](int s, int o) {
+                if constexpr (cut) mask.put(m[s], e0, o);
+                G.put(x[s], 8 * e0, 8 * o);
+            });
         };
         xfft<P, -1, BL>(v, tw, t, L, bl, g0, none, stX);
     } else if constexpr (K == RK_MID) {
-        cf *G = (cf *) a.G + wb;
-        const uint8_t *mask = a.mask + wb;
         const float beta = a.beta;
         cf g[P::E];
         uint8_t m[P::E];
+        auto ldX = ld(X);
         auto pre = [&](const auto &el) {
-            el.load([&](int s, int o, int d) {
-                g[s] = at32(G + o, lr + d);
-                m[s] = at32(mask + o, lr + d);
+            el.load([&](int s, int o) {
+                g[s] = G.get<cf>(8 * e0, 8 * o);
+                m[s] = mask.get<uint8_t>(e0, o);
             });
         };
         auto mid = [&](auto &x, const auto &el) {
-            el.all([&](int s, int o) { x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta); });
-            if (valid) el.store([&](int s, int o, int d) { at32(G + o, lr + d) = x[s]; });
+            el.load([&](int s, int) { x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta); });
+            if (valid) el.store([&](int s, int o) { G.put(x[s], 8 * e0, 8 * o); });
         };
-        xpair<P, +1, -1, BL, PF>(v, tw, t, L, bl, ldX, pre, mid, stX);
+        xpair<P, +1, -1, BL, WHEN>(v, tw, t, L, bl, ldX, pre, mid, stX);
     }
 }
 
@@ -187,26 +178,27 @@ constexpr int kInitErr = kRowWriteG | kRowWriteBn | kRowError;
 template <int NL>
 constexpr size_t row_lds(int n) { return sizeof(cf) * (size_t) NL * lds_elems(n); }
 
-template <class P, int NL, bool PF = false, bool BL = false, int STG = 0>
+template <class P, int NL, int WHEN = kAtJunction, bool BL = false>
 int launch_variant(int mode, RowArgs a, hipStream_t s)
 {
     static_assert(NL * P::T <= 1024, "row workgroup too large");
     const dim3 grid((a.H + NL - 1) / NL, a.batch > 1 ? a.batch : 1), block(NL * P::T);
     constexpr size_t lds = row_lds<NL>(P::n);
     static_assert(lds <= kLdsBudget, "row tile exceeds the LDS budget");
+    constexpr int AJ = kAtJunction;
     if constexpr (lds > 64 * 1024) {
         static const hipError_t attr = [&] {
             hipError_t e = hipSuccess;
-            for (const void *f : {(const void *) k_row<P, NL, RK_FWD, false, BL>,
-                                  (const void *) k_row<P, NL, RK_FWD_NORM, false, BL>,
-                                  (const void *) k_row<P, NL, RK_INV, false, BL>,
-                                  (const void *) k_row<P, NL, RK_INVOUT, false, BL, 0, kInit>,
-                                  (const void *) k_row<P, NL, RK_INVOUT, false, BL, 0, kLast>,
-                                  (const void *) k_row<P, NL, RK_INVOUT, false, BL, 0, 0>,
-                                  (const void *) k_row<P, NL, RK_INVOUT, false, BL, 0, kInitErr>,
-                                  (const void *) k_row<P, NL, RK_FIRST, false, BL, 0, kRowCut>,
-                                  (const void *) k_row<P, NL, RK_FIRST, false, BL, 0, 0>,
-                                  (const void *) k_row<P, NL, RK_MID, PF, BL, STG>})
+            for (const void *f : {(const void *) k_row<P, NL, RK_FWD, AJ, BL>,
+                                  (const void *) k_row<P, NL, RK_FWD_NORM, AJ, BL>,
+                                  (const void *) k_row<P, NL, RK_INV, AJ, BL>,
+                                  (const void *) k_row<P, NL, RK_INVOUT, AJ, BL, kInit>,
+                                  (const void *) k_row<P, NL, RK_INVOUT, AJ, BL, kLast>,
+                                  (const void *) k_row<P, NL, RK_INVOUT, AJ, BL, 0>,
+                                  (const void *) k_row<P, NL, RK_INVOUT, AJ, BL, kInitErr>,
+                                  (const void *) k_row<P, NL, RK_FIRST, AJ, BL, kRowCut>,
+                                  (const void *) k_row<P, NL, RK_FIRST, AJ, BL, 0>,
+                                  (const void *) k_row<P, NL, RK_MID, WHEN, BL>})
                 if (e == hipSuccess)
                     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
             return e;
@@ -214,114 +206,74 @@ int launch_variant(int mode, RowArgs a, hipStream_t s)
         if (attr != hipSuccess) return from_hip(attr);
     }
     switch (mode) {
-    case ROW_FWD: IMR_LAUNCH((k_row<P, NL, RK_FWD, false, BL>), grid, block, lds, s, a); break;
-    case ROW_FWD_NORM: IMR_LAUNCH((k_row<P, NL, RK_FWD_NORM, false, BL>), grid, block, lds, s, a); break;
-    case ROW_INV: IMR_LAUNCH((k_row<P, NL, RK_INV, false, BL>), grid, block, lds, s, a); break;
-    case ROW_INIT: IMR_LAUNCH((k_row<P, NL, RK_INVOUT, false, BL, 0, kInit>), grid, block, lds, s, a); break;
-    case ROW_LAST: IMR_LAUNCH((k_row<P, NL, RK_INVOUT, false, BL, 0, kLast>), grid, block, lds, s, a); break;
-    case ROW_LAST_PLAIN: IMR_LAUNCH((k_row<P, NL, RK_INVOUT, false, BL, 0, 0>), grid, block, lds, s, a); break;
-    case ROW_INIT_ERR:
-        IMR_LAUNCH((k_row<P, NL, RK_INVOUT, false, BL, 0, kInitErr>), grid, block, lds, s, a);
-        break;
-    case ROW_FIRST_CUT: IMR_LAUNCH((k_row<P, NL, RK_FIRST, false, BL, 0, kRowCut>), grid, block, lds, s, a); break;
-    case ROW_FIRST_MASK: IMR_LAUNCH((k_row<P, NL, RK_FIRST, false, BL, 0, 0>), grid, block, lds, s, a); break;
-    case ROW_MID: IMR_LAUNCH((k_row<P, NL, RK_MID, PF, BL, STG>), grid, block, lds, s, a); break;
+    case ROW_FWD: IMR_LAUNCH((k_row<P, NL, RK_FWD, AJ, BL>), grid, block, lds, s, a); break;
+    case ROW_FWD_NORM: IMR_LAUNCH((k_row<P, NL, RK_FWD_NORM, AJ, BL>), grid, block, lds, s, a); break;
+    case ROW_INV: IMR_LAUNCH((k_row<P, NL, RK_INV, AJ, BL>), grid, block, lds, s, a); break;
+    case ROW_INIT: IMR_LAUNCH((k_row<P, NL, RK_INVOUT, AJ, BL, kInit>), grid, block, lds, s, a); break;
+    case ROW_LAST: IMR_LAUNCH((k_row<P, NL, RK_INVOUT, AJ, BL, kLast>), grid, block, lds, s, a); break;
+    case ROW_LAST_PLAIN: IMR_LAUNCH((k_row<P, NL, RK_INVOUT, AJ, BL, 0>), grid, block, lds, s, a); break;
+    case ROW_INIT_ERR: IMR_LAUNCH((k_row<P, NL, RK_INVOUT, AJ, BL, kInitErr>), grid, block, lds, s, a); break;
+    case ROW_FIRST_CUT: IMR_LAUNCH((k_row<P, NL, RK_FIRST, AJ, BL, kRowCut>), grid, block, lds, s, a); break;
+    case ROW_FIRST_MASK: IMR_LAUNCH((k_row<P, NL, RK_FIRST, AJ, BL, 0>), grid, block, lds, s, a); break;
+    case ROW_MID: IMR_LAUNCH((k_row<P, NL, RK_MID, WHEN, BL>), grid, block, lds, s, a); break;
     default: return IMRESH_ERR_INVALID;
     }
     return imr::launch_status(__FILE__, __LINE__);
 }
 
-// Row variants of a length (index: workgroup shape, then +count/2 for the
-// prefetching RK_MID): shapes 0 = E 16 with ~256-thread groups; for long
-// rows also 1 = E 32 (half the threads per row), 2 = E 16 with twice the
-// rows, 3 = shape 0 with the second half of the grid started ~3.4 us late and,
-// when a group holds 2 or more rows, a last shape with half the rows: fewer
-// waves share each barrier, so the groups of a CU drift out of phase and
-// overlap one's loads with another's arithmetic (2048^2: 23.8 -> 22.6 us);
-// for short lines (<= 512 points, >= 8 rows per group) 1 = a quarter of the
-// rows per group: 4x the workgroups, which spreads one small image over more
-// CUs (a 256^2 reconstruction 199 -> 227 per second).
-template <int N>
-constexpr bool long_pow2() { return N >= 1024 && (N & (N - 1)) == 0; }
-
-// shapes 0-3 of the long power-of-two lengths (2 when twice the rows do
-// not fit a workgroup)
+// Row variants of a length: index = when * shapes + shape.  `when` is where
+// RK_MID reads gPrev and the mask (line_pair); shape 0 has ~256-thread
+// groups, shape 1 fewer rows per group: half of them for 1024 and 2048
+// points (fewer waves share each barrier, so the groups of a CU drift out of
+// phase and overlap one's loads with another's arithmetic), a quarter for up
+// to 512 points (4x the workgroups spread one small image over more CUs).
 template <int N, int... Rs>
-constexpr int long_row_shapes()
+constexpr int small_group()
 {
-    using P16 = PlanE<16, N, Rs...>;
-    return (2 * P16::L * P16::T <= 1024 &&
-            row_lds<2 * P16::L>(N) <= kLdsBudget) ? 4 : 2;
+    using P = Plan<N, Rs...>;
+    if (N <= 512 && P::L >= 8) return P::L / 4;
+    if (N >= 1024 && (N & (N - 1)) == 0 && P::L >= 2) return P::L / 2;
+    return 0;
 }
 
 template <int N, int... Rs>
-constexpr int row_shape_count()
-{
-    using P16 = PlanE<16, N, Rs...>;
-    if constexpr (long_pow2<N>()) {   // extra shapes for the long power-of-two lengths
-        return long_row_shapes<N, Rs...>() + (P16::L >= 2 ? 1 : 0);   // + half the rows
-    } else if constexpr (N <= 512 && P16::L >= 8) {
-        return 2;   // short lines: also groups of a quarter of the rows (4x the workgroups)
-    }
-    return 1;
-}
+constexpr int row_shape_count() { return small_group<N, Rs...>() > 0 ? 2 : 1; }
 
 template <int N, int... Rs>
-constexpr int row_variant_count() { return 2 * row_shape_count<N, Rs...>(); }
+constexpr int row_variant_count() { return 3 * row_shape_count<N, Rs...>(); }
 
-// Bluestein kernels exist for the power-of-two convolution lengths
+// Bluestein kernels exist for the power-of-two convolution lengths, with half
+// the plan's rows per group (a mid-size image over more CUs)
 template <int N>
 constexpr bool blue_length() { return N >= 64 && N <= 2 * kMaxLine && (N & (N - 1)) == 0; }
 
-template <class P, int NL, int STG = 0>
-int launch_pf(bool pf, int mode, RowArgs a, hipStream_t s)
-{
-    return pf ? launch_variant<P, NL, true, false, STG>(mode, a, s)
-              : launch_variant<P, NL, false, false, STG>(mode, a, s);
-}
+template <class P>
+constexpr int blue_rows() { return P::L > 1 ? P::L / 2 : 1; }
 
-template <int N, int... Rs>
-int launch_row_direct(int var, int mode, RowArgs a, hipStream_t s);
+template <class P, int NL>
+int launch_when(int when, int mode, RowArgs a, hipStream_t s)
+{
+    if (when == kEarly) return launch_variant<P, NL, kEarly>(mode, a, s);
+    if (when == kAhead) return launch_variant<P, NL, kAhead>(mode, a, s);
+    return launch_variant<P, NL>(mode, a, s);
+}
 
 template <int N, int... Rs>
 int launch_row_variant(int var, int mode, RowArgs a, hipStream_t s)
 {
-    using P16 = PlanE<16, N, Rs...>;
+    using P = Plan<N, Rs...>;
     if constexpr (blue_length<N>()) {
-        if (var == kBlueVariant) return launch_variant<P16, P16::L, false, true>(mode, a, s);
-        if (var == kBlueVariant + 1) return launch_variant<P16, P16::L, true, true>(mode, a, s);
-        if (var == kBlueVariant + 2)
-            return launch_variant<P16, (P16::L > 1 ? P16::L / 2 : 1), false, true>(mode, a, s);
+        if (var == kBlueVariant) return launch_variant<P, blue_rows<P>(), kAtJunction, true>(mode, a, s);
     }
     if constexpr (N > kMaxLine) {
         return IMRESH_ERR_UNSUPPORTED_SIZE;   // a convolution length only
     } else {
-        return launch_row_direct<N, Rs...>(var, mode, a, s);
-    }
-}
-
-template <int N, int... Rs>
-int launch_row_direct(int var, int mode, RowArgs a, hipStream_t s)
-{
-    using P16 = PlanE<16, N, Rs...>;
-    constexpr int ns = row_shape_count<N, Rs...>();
-    const bool pf = var >= ns;
-    const int shape = pf ? var - ns : var;
-    if constexpr (long_pow2<N>() && ns > 1) {
-        using P32 = PlanE<32, N, Rs...>;
-        if (shape == 1) return launch_pf<P32, P32::L>(pf, mode, a, s);
-        constexpr int nb = long_row_shapes<N, Rs...>();
-        if constexpr (nb == 4) {
-            if (shape == 2) return launch_pf<P16, 2 * P16::L>(pf, mode, a, s);
-            if (shape == 3) return launch_pf<P16, P16::L, 1>(pf, mode, a, s);
+        constexpr int ns = row_shape_count<N, Rs...>();
+        if constexpr (ns > 1) {
+            if (var % ns == 1) return launch_when<P, small_group<N, Rs...>()>(var / ns, mode, a, s);
         }
-        if constexpr (ns > nb) {
-            if (shape == nb) return launch_pf<P16, P16::L / 2>(pf, mode, a, s);
-        }
-    } else if constexpr (ns > 1) {
-        if (shape == 1) return launch_pf<P16, P16::L / 4>(pf, mode, a, s);
+        return launch_when<P, P::L>(var / ns, mode, a, s);
     }
-    return launch_pf<P16, P16::L>(pf, mode, a, s);
 }
 
 // rows per workgroup of a variant (the host needs it for the partial sums;
@@ -329,21 +281,10 @@ int launch_row_direct(int var, int mode, RowArgs a, hipStream_t s)
 template <int N, int... Rs>
 int row_variant_rows(int var)
 {
-    using P16 = PlanE<16, N, Rs...>;
-    if (var == kBlueVariant + 2) return P16::L > 1 ? P16::L / 2 : 1;
-    if (var >= kBlueVariant) return P16::L;
+    using P = Plan<N, Rs...>;
+    if (var == kBlueVariant) return blue_rows<P>();
     constexpr int ns = row_shape_count<N, Rs...>();
-    const int shape = var >= ns ? var - ns : var;
-    if constexpr (long_pow2<N>() && ns > 1) {
-        using P32 = PlanE<32, N, Rs...>;
-        constexpr int nb = long_row_shapes<N, Rs...>();
-        if (shape == 1) return P32::L;
-        if (nb == 4 && shape == 2) return 2 * P16::L;
-        if (ns > nb && shape == nb) return P16::L / 2;
-    } else if constexpr (ns > 1) {
-        if (shape == 1) return P16::L / 4;
-    }
-    return P16::L;
+    return var % ns == 1 ? small_group<N, Rs...>() : P::L;
 }
 
 template <int G, int N, int... Rs>

@@ -53,16 +53,19 @@ template <int E, class El>
 __device__ __forceinline__ void modulus_project_line(cf (&v)[E], const float (&m)[E], const El &el)
 {
     float low = 1e-30f;
-    el.all([&](int s, int o) {
+    el.load([&](int s, int o) {
         const float n2 = v[s].x * v[s].x + v[s].y * v[s].y;
         if (el.inside(o)) low = fminf(low, n2);
     });
     if (low >= 1e-30f) {
-        el.all([&](int s, int) {
-            v[s] = modulus_project_fast(v[s], v[s].x * v[s].x + v[s].y * v[s].y, m[s]);
+        // (elements past the end of a line are 0 and have to stay finite)
+        el.load([&](int s, int) {
+            float n2 = v[s].x * v[s].x + v[s].y * v[s].y;
+            if constexpr (El::span < El::Q::nb * El::Q::R) n2 = fmaxf(n2, 1e-30f);
+            v[s] = modulus_project_fast(v[s], n2, m[s]);
         });
     } else {
-        el.all([&](int s, int) {
+        el.load([&](int s, int) {
             const float n2 = v[s].x * v[s].x + v[s].y * v[s].y;
             v[s] = n2 >= 1e-30f ? modulus_project_fast(v[s], n2, m[s]) : modulus_project(v[s], m[s]);
         });

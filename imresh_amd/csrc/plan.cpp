@@ -140,8 +140,9 @@ std::vector<float2> blue_tables(int n, int m)
     dft_any(bf);
     dft_any(bi);
     std::vector<float2> out;
-    out.reserve((size_t) n + 2 * m);
+    out.reserve((size_t) m / 2 + 2 * m);
     for (int j = 0; j < n; ++j) out.push_back(make_float2((float) a[j].real(), (float) a[j].imag()));
+    out.resize((size_t) m / 2, make_float2(0.f, 0.f));
     for (int k = 0; k < m; ++k) out.push_back(make_float2((float) (bf[k].real() / m), (float) (bf[k].imag() / m)));
     for (int k = 0; k < m; ++k) out.push_back(make_float2((float) (bi[k].real() / m), (float) (bi[k].imag() / m)));
     return out;
@@ -299,7 +300,7 @@ int row_grid(const Plan2D &p)
 {
     int L = 1;
     const int n = p.row.blue ? p.row.m : p.W;
-    const int v = p.row.blue ? kBlueVariant + kBlueRowDefault : p.rowVar;
+    const int v = p.row.blue ? kBlueVariant : p.rowVar;
     switch (p.row.group) {
     case 0: L = row_rows_g0(n, v); break;
     case 1: L = row_rows_g1(n, v); break;
@@ -320,7 +321,7 @@ int launch_row(int mode, const Plan2D &p, RowArgs a, hipStream_t s)
     a.len = p.W;
     a.bs = p.row.bs;
     const int n = p.row.blue ? p.row.m : p.W;
-    const int v = p.row.blue ? kBlueVariant + kBlueRowDefault : p.rowVar;
+    const int v = p.row.blue ? kBlueVariant : p.rowVar;
     switch (p.row.group) {
     case 0: return launch_row_g0(mode, v, n, p.row, a, s);
     case 1: return launch_row_g1(mode, v, n, p.row, a, s);
@@ -360,7 +361,7 @@ int launch_col_fourstep(const Plan2D &p, ColArgs a, hipStream_t s)
     Plan2D q = p;
     q.H = h2;
     IMR_CHECK(get_line_plan(dev, h2, &q.col));
-    q.colVar = col_variants(q.col) / 2;   // the prefetching default tile
+    q.colVar = col_variants(q.col) / 3 * 2;   // the plan's tile, modulus read early
     ColArgs b = a;
     b.batch = images;
     b.sub = 8;
@@ -381,7 +382,7 @@ int launch_col(int mode, const Plan2D &p, ColArgs a, hipStream_t s)
     a.len = p.H;
     a.bs = p.col.bs;
     const int n = p.col.blue ? p.col.m : p.H;
-    const int v = p.col.blue ? kBlueVariant + kBlueColDefault : p.colVar;
+    const int v = p.col.blue ? kBlueVariant : p.colVar;
     switch (p.col.group) {
     case 0: return launch_col_g0(mode, v, n, p.col, a, s);
     case 1: return launch_col_g1(mode, v, n, p.col, a, s);
@@ -397,7 +398,7 @@ int launch_col(int mode, const Plan2D &p, ColArgs a, hipStream_t s)
 
 int row_variants(const LinePlan &lp)
 {
-    if (lp.blue) return 1;   // Bluestein: fixed choice (no per-size tuning, see kBlueColDefault)
+    if (lp.blue) return 1;   // Bluestein: fixed choice (see kBlueVariant)
     switch (lp.group) {
     case 0: return row_variants_g0(lp.n);
     case 1: return row_variants_g1(lp.n);
