@@ -95,15 +95,25 @@ int ws_alloc(int device, int W, int H, Workspace **out)
         return from_hip(e);
     }
     ws_layout(w, W, H, base);
-    e = hipHostMalloc((void **) &w->host_stage, 4096, hipHostMallocDefault);
+    e = hipHostMalloc((void **) &w->host_stage, 4096, hipHostMallocCoherent);
     if (e != hipSuccess) {
         (void) hipFree(w->base);
         if (w->host_stage) (void) hipHostFree(w->host_stage);
         delete w;
         return from_hip(e);
     }
+    w->done_word = (uint32_t *) w->host_stage + 512;   // its own part of the pinned block
+    *w->done_word = 0;
     *out = w;
     return IMRESH_OK;
+}
+
+bool ws_busy(Workspace *w)
+{
+    if (!w->busy.load(std::memory_order_acquire)) return false;
+    if (__atomic_load_n(w->done_word, __ATOMIC_ACQUIRE) != w->done_seq) return true;
+    w->busy.store(false, std::memory_order_release);
+    return false;
 }
 
 void ws_release(Workspace *w)
@@ -120,7 +130,7 @@ void ws_release(Workspace *w)
 bool ws_wait_idle(Workspace *w, double timeout_s)
 {
     const auto t0 = std::chrono::steady_clock::now();
-    while (w->busy.load(std::memory_order_acquire)) {
+    while (ws_busy(w)) {
         if (std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > timeout_s)
             return false;
         std::this_thread::sleep_for(std::chrono::microseconds(20));
@@ -169,7 +179,7 @@ void trim_idle(size_t cap, std::vector<Workspace *> &out)
         for (auto &kv : g_ws_free)
             for (size_t i = 0; i < kv.second.size(); ++i) {
                 Workspace *w = kv.second[i];
-                if (w->busy.load(std::memory_order_acquire)) continue;
+                if (ws_busy(w)) continue;
                 if (lru == nullptr || w->last_use < lru->last_use) {
                     lru = w;
                     list = &kv.second;
@@ -191,7 +201,7 @@ int ws_checkout(int device, int W, int H, hipStream_t s, Workspace **out)
         std::lock_guard<std::mutex> lk(g_ws_mtx);
         auto &v = g_ws_free[{device, W, H}];
         for (size_t i = 0; i < v.size() && w == nullptr; ++i)
-            if (!v[i]->busy.load(std::memory_order_acquire)) {
+            if (!ws_busy(v[i])) {
                 w = v[i];
                 v.erase(v.begin() + (long) i);
             }
@@ -238,19 +248,18 @@ int ws_checkout(int device, int W, int H, hipStream_t s, Workspace **out)
     return IMRESH_OK;
 }
 
-void mark_idle(void *p) { static_cast<Workspace *>(p)->busy.store(false, std::memory_order_release); }
-
 // synced: the caller has synchronized the stream after its last use of
-// the workspace (then it is idle at once; otherwise a host function behind
-// the queued work marks it idle)
+// the workspace (then it is idle at once; otherwise its completion word,
+// stored behind the queued work, tells)
 void ws_return(Workspace *w, hipStream_t s, bool synced = false)
 {
     if (synced) {
         w->busy.store(false, std::memory_order_release);
     } else {
-        w->busy.store(true, std::memory_order_relaxed);
-        if (hipLaunchHostFunc(s, mark_idle, w) != hipSuccess) {
-            (void) hipStreamSynchronize(s);   // no host function: wait here instead
+        ++w->done_seq;
+        w->busy.store(true, std::memory_order_release);
+        if (launch_signal(w->done_word, w->done_seq, s) != IMRESH_OK) {
+            (void) hipStreamSynchronize(s);   // nothing will tell: wait here instead
             w->busy.store(false, std::memory_order_release);
         }
     }
@@ -492,6 +501,17 @@ RowArgs row_args(const Workspace *w, const Params &q)
 }
 }  // namespace
 
+// the scalars and the flags lie kStageFlags floats apart in the workspace
+// allocation (each region 256-byte aligned), so one kernel resets or stages
+// both
+constexpr size_t kStageFlags = 64;
+
+static int reset_state(Workspace *w, hipStream_t s)
+{
+    if ((const void *) w->flags != (const void *) (w->scal + kStageFlags)) return IMRESH_ERR_INTERNAL;
+    return launch_zero_words(w->scal, kStageFlags + 16, s);
+}
+
 int ws_tune(Workspace *w, hipStream_t s) { return autotune(w->device, w->W, w->H, s, w); }
 
 int recon_begin(Workspace *w, const float *M, const Params &q, hipStream_t s)
@@ -499,8 +519,7 @@ int recon_begin(Workspace *w, const float *M, const Params &q, hipStream_t s)
     IMR_CHECK(ensure_weights(w, q, s));
     if (M != w->M)
         IMR_HIP_CHECK(hipMemcpyAsync(w->M, M, sizeof(float) * w->n, hipMemcpyDeviceToDevice, s));
-    IMR_HIP_CHECK(hipMemsetAsync(w->flags, 0, 64, s));
-    IMR_HIP_CHECK(hipMemsetAsync(w->scal, 0, 64, s));
+    IMR_CHECK(reset_state(w, s));
     Plan2D p;
     IMR_CHECK(get_plan2d(w->device, w->W, w->H, &p));
     IMR_CHECK(launch_col(COL_INIT, p, col_args(w, w->M), s));
@@ -625,17 +644,11 @@ int recon_end(Workspace *w, float *io_dev, hipStream_t s)
     return launch_copy_from_real(io_dev, w->X, w->n, s);
 }
 
-// the scalars and the flags lie kStageFlags floats apart in the workspace
-// allocation (each region 256-byte aligned), so one copy stages both
-constexpr size_t kStageFlags = 64;
-
 int recon_stage_results(Workspace *w, hipStream_t s)
 {
     static_assert(sizeof(float) * (kStageFlags + 2) <= 4096, "staging buffer");
     if ((const void *) w->flags != (const void *) (w->scal + kStageFlags)) return IMRESH_ERR_INTERNAL;
-    IMR_HIP_CHECK(hipMemcpyAsync(w->host_stage, w->scal, sizeof(float) * (kStageFlags + 2),
-                                 hipMemcpyDeviceToHost, s));
-    return IMRESH_OK;
+    return launch_stage_words(w->host_stage, w->scal, kStageFlags + 2, s);
 }
 
 void recon_read_staged(const Workspace *w, imresh_result *res, int *done)
@@ -676,8 +689,8 @@ hipStream_t S(void *s) { return (hipStream_t) s; }
 
 // Device scratch of the asynchronous per-operator entry points (the blur's
 // temporary plane, the Poisson simulation's sums), pooled per device: a
-// buffer is held by its call, then stays busy until a host function behind
-// the call's work on the caller's stream frees it.  (Stream-ordered
+// buffer is held by its call, then stays busy until its completion word,
+// stored behind the call's work on the caller's stream, holds its value.  (Stream-ordered
 // allocation would leave the allocator tracking the caller's stream, which
 // the caller may destroy.)
 struct PoolBuf {
@@ -685,11 +698,19 @@ struct PoolBuf {
     size_t bytes = 0;
     int dev = 0;
     std::atomic<int> state{0};   // 0 free, 1 held by a call, 2 busy on a stream
+    uint32_t *word = nullptr;    // coherent host memory
+    uint32_t seq = 0;
+
+    // takes a buffer that is free, or whose last work has run
+    bool take()
+    {
+        int st = state.load(std::memory_order_acquire);
+        if (st == 2 && __atomic_load_n(word, __ATOMIC_ACQUIRE) != seq) return false;
+        return st != 1 && state.compare_exchange_strong(st, 1);
+    }
 };
 std::mutex g_pb_mtx;
 std::vector<PoolBuf *> g_pb;
-
-void pool_buf_free(void *p) { static_cast<PoolBuf *>(p)->state.store(0, std::memory_order_release); }
 
 struct Scratch {
     void *p = nullptr;
@@ -703,8 +724,7 @@ struct Scratch {
         {
             std::lock_guard<std::mutex> lk(g_pb_mtx);
             for (PoolBuf *x : g_pb) {
-                int fr = 0;
-                if (x->dev == dev && x->bytes >= bytes && x->state.compare_exchange_strong(fr, 1)) {
+                if (x->dev == dev && x->bytes >= bytes && x->take()) {
                     b = x;
                     break;
                 }
@@ -717,11 +737,16 @@ struct Scratch {
             x->bytes = cap;
             x->dev = dev;
             x->state.store(1);
-            const hipError_t e = hipMalloc(&x->p, cap);
+            hipError_t e = hipMalloc(&x->p, cap);
+            if (e == hipSuccess) {
+                e = hipHostMalloc((void **) &x->word, 64, hipHostMallocCoherent);
+                if (e != hipSuccess) (void) hipFree(x->p);
+            }
             if (e != hipSuccess) {
                 delete x;
                 return IMR_HIP_STATUS(e);
             }
+            *x->word = 0;
             std::lock_guard<std::mutex> lk(g_pb_mtx);
             g_pb.push_back(x);
             b = x;
@@ -732,9 +757,11 @@ struct Scratch {
     ~Scratch()
     {
         if (b == nullptr) return;
-        b->state.store(2, std::memory_order_relaxed);
-        if (hipLaunchHostFunc(s, pool_buf_free, b) != hipSuccess) {
-            (void) hipStreamSynchronize(s);   // no host function: wait here instead
+        ++b->seq;
+        if (launch_signal(b->word, b->seq, s) == IMRESH_OK) {
+            b->state.store(2, std::memory_order_release);
+        } else {
+            (void) hipStreamSynchronize(s);   // nothing will tell: wait here instead
             b->state.store(0, std::memory_order_release);
         }
     }
@@ -748,14 +775,14 @@ void pool_bufs_release()
         std::lock_guard<std::mutex> lk(g_pb_mtx);
         std::vector<PoolBuf *> keep;
         for (PoolBuf *x : g_pb) {
-            int fr = 0;
-            if (x->state.compare_exchange_strong(fr, 1)) drop.push_back(x);
+            if (x->take()) drop.push_back(x);
             else keep.push_back(x);
         }
         g_pb.swap(keep);
     }
     for (PoolBuf *x : drop) {
         (void) hipFree(x->p);
+        (void) hipHostFree(x->word);
         delete x;
     }
 }
@@ -765,7 +792,8 @@ size_t pool_bufs_bytes()
     std::lock_guard<std::mutex> lk(g_pb_mtx);
     size_t t = 0;
     for (PoolBuf *x : g_pb)
-        if (x->state.load() == 0) t += x->bytes;
+        if (x->state.load() != 1 && (x->state.load() == 0 || __atomic_load_n(x->word, __ATOMIC_ACQUIRE) == x->seq))
+            t += x->bytes;
     return t;
 }
 
@@ -802,7 +830,7 @@ int reduce_slot_get(int dev, ReduceSlot *out)
     }
     ReduceSlot r;
     IMR_HIP_CHECK(hipMalloc(&r.dev, kReduceSlotBytes));
-    const hipError_t e = hipHostMalloc((void **) &r.host, 64, hipHostMallocDefault);
+    const hipError_t e = hipHostMalloc((void **) &r.host, 64, hipHostMallocCoherent);
     if (e != hipSuccess) {
         (void) hipFree(r.dev);
         return from_hip(e);
@@ -872,9 +900,8 @@ int vector_reduce(int op, const float *d, uint32_t n, float *out, void *stream)
     hipStream_t s = S(stream);
     SlotHold sh;
     IMR_CHECK(sh.take(s));
-    float *part = (float *) sh.r.dev, *res = part + kReduceBlocks;
-    IMR_CHECK(launch_reduce(op, d, n, part, kReduceBlocks, res, s));
-    IMR_HIP_CHECK(hipMemcpyAsync(sh.r.host, res, sizeof(float), hipMemcpyDeviceToHost, s));
+    // the last kernel stores the result in the slot's pinned host block
+    IMR_CHECK(launch_reduce(op, d, n, (float *) sh.r.dev, kReduceBlocks, sh.r.host, s));
     IMR_HIP_CHECK(hipStreamSynchronize(s));
     sh.done = true;
     *out = sh.r.host[0];
@@ -890,10 +917,8 @@ int hio_error(const float *g, const void *mask, int kind, uint32_t n, int invert
     IMR_CHECK(sh.take(s));
     float *perr = (float *) sh.r.dev;
     unsigned *pcnt = (unsigned *) (perr + kReduceBlocks);
-    float *res = perr + 2 * kReduceBlocks;
     IMR_CHECK(launch_hio_error((const float2 *) g, mask, kind, n, invert, perr, pcnt, kReduceBlocks,
-                               res, s));
-    IMR_HIP_CHECK(hipMemcpyAsync(sh.r.host, res, 3 * sizeof(float), hipMemcpyDeviceToHost, s));
+                               sh.r.host, s));
     IMR_HIP_CHECK(hipStreamSynchronize(s));
     sh.done = true;
     const float *h = sh.r.host;
@@ -1324,8 +1349,7 @@ int run_hio_standalone(Workspace *w, unsigned n_cycles, float target, float beta
     cf.out = w->X;
     IMR_CHECK(launch_col(COL_FWD, p, cf, s));
     IMR_CHECK(launch_random_phase(w->X, w->M, n, s));
-    IMR_HIP_CHECK(hipMemsetAsync(w->flags, 0, 64, s));
-    IMR_HIP_CHECK(hipMemsetAsync(w->scal, 0, 64, s));
+    IMR_CHECK(reset_state(w, s));
     // first inverse transform; gPrevious = g' (:238-239)
     cf.in = w->X;
     IMR_CHECK(launch_col(COL_INV, p, cf, s));

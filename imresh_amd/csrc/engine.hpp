@@ -46,11 +46,14 @@ struct Workspace {
     size_t host_wpin_n = 0;            // its capacity in floats
     float *host_stage = nullptr;  // pinned, 64 floats + readback
     // set when a user returns the workspace with work still queued on its
-    // stream, cleared by a host function enqueued behind that work.  (An
-    // event recorded on the user's stream would do, but HIP reads the
-    // stream an event was last recorded on when the event is queried or
-    // waited for, and the caller may have destroyed that stream by then.)
+    // stream; the work has run once done_word (pinned, stored by a kernel
+    // queued behind it) holds done_seq.  (An event recorded on the user's
+    // stream would do, but HIP reads the stream an event was last recorded on
+    // when the event is queried or waited for, and the caller may have
+    // destroyed that stream by then.)
     std::atomic<bool> busy{false};
+    uint32_t *done_word = nullptr;
+    uint32_t done_seq = 0;
     uint64_t last_use = 0;        // pool clock of the last return (idle trimming)
     // the captured cycle graph and the parameters it was captured with
     hipGraphExec_t gexec = nullptr;
@@ -64,6 +67,8 @@ struct Workspace {
 // returns the bytes the layout needs
 size_t ws_layout(Workspace *w, int W, int H, void *base);
 int ws_alloc(int device, int W, int H, Workspace **out);
+// work of the workspace's previous user still queued or running
+bool ws_busy(Workspace *w);
 // blocks the calling thread until the workspace's previous user's work has
 // run (no-op for an idle workspace); false after timeout_s seconds
 bool ws_wait_idle(Workspace *w, double timeout_s);

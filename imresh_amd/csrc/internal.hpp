@@ -217,7 +217,7 @@ int launch_apply_modulus(float2 *out, const float2 *in, const float *M, size_t n
 int launch_hio_constraint(float2 *gp, const float2 *g, const float *mask, size_t n, float beta,
                           hipStream_t s);
 int launch_cutoff(float *d, size_t n, float t, float lo, float hi, hipStream_t s);
-// op: 0 = max, 1 = min, 2 = sum.  result: device float.
+// op: 0 = max, 1 = min, 2 = sum.  result: device or pinned host float.
 int launch_reduce(int op, const float *d, size_t n, float *partials, int np, float *result,
                   hipStream_t s);
 // mask kinds of launch_hio_error
@@ -232,6 +232,13 @@ int launch_fill_state(float2 *X, float2 *G, uint8_t *mask, float *M, float *Bn, 
 // kernel arguments, kStoreWords per launch: no staging buffer, capturable
 constexpr int kStoreWords = 480;
 int launch_store_words(float *dst, const float *src, size_t n, hipStream_t s);
+
+// value -> word (coherent host memory) once the work queued before it has run
+int launch_signal(uint32_t *word, uint32_t value, hipStream_t s);
+// n zero words; n words of device memory to pinned host memory (single small
+// kernels: a memset or copy of a few words costs the stream more)
+int launch_zero_words(float *d, unsigned n, hipStream_t s);
+int launch_stage_words(float *host, const float *d, unsigned n, hipStream_t s);
 
 constexpr int kReduceBlocks = 512;
 constexpr int kBlurTX = 64;

@@ -387,7 +387,44 @@ __global__ void k_store_words(float *dst, unsigned n, StoreWords a)
     for (unsigned i = threadIdx.x; i < n; i += blockDim.x) dst[i] = a.v[i];
 }
 
+// Completion word of a pooled buffer: a value in coherent host memory, stored
+// behind the work that uses the buffer.  One thread, ~2 us on the stream; a
+// host function there held the stream until a host thread had woken and run
+// it (forward model and blur calls: see launch_signal).
+__global__ void k_signal(uint32_t *word, uint32_t value)
+{
+    __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void __launch_bounds__(256) k_zero_words(float *d, unsigned n)
+{
+    for (unsigned i = threadIdx.x; i < n; i += blockDim.x) d[i] = 0.f;
+}
+
+__global__ void __launch_bounds__(128) k_stage_words(float *host, const float *d, unsigned n)
+{
+    for (unsigned i = threadIdx.x; i < n; i += blockDim.x) host[i] = d[i];
+}
+
 // ------------------------------------------------------------ launchers
+int launch_signal(uint32_t *word, uint32_t value, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_signal, dim3(1), dim3(1), 0, s, word, value);
+    return imr::launch_status(__FILE__, __LINE__);
+}
+
+int launch_zero_words(float *d, unsigned n, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(256), 0, s, d, n);
+    return imr::launch_status(__FILE__, __LINE__);
+}
+
+int launch_stage_words(float *host, const float *d, unsigned n, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_stage_words, dim3(1), dim3(128), 0, s, host, d, n);
+    return imr::launch_status(__FILE__, __LINE__);
+}
+
 static int grid_1d(size_t n)
 {
     size_t g = (n + 255) / 256;
