@@ -46,20 +46,8 @@ __device__ __forceinline__ void blue_apply_chirp(cf (&v)[PM::E], const cf (&ch)[
     el.all([&](int s, int) { v[s] = cmul(v[s], DIR < 0 ? ch[s] : mkc(ch[s].x, -ch[s].y)); });
 }
 
-// the plan's elements past the span of a line
-template <class PM, class El>
-__device__ __forceinline__ void blue_pad(cf (&v)[PM::E])
-{
-    using Q = typename El::Q;
-#pragma unroll
-    for (int b = 0; b < Q::B; ++b)
-#pragma unroll
-        for (int r = 0; r < Q::R; ++r)
-            if (b * Q::T + r * Q::nb >= El::span) v[b * Q::R + r] = mkc(0.f, 0.f);
-}
-
-// circular convolution with the chirp: v holds the chirped, zero-padded
-// line at PM's forward first-pass input positions on entry and the result
+// circular convolution with the chirp: v holds the chirped line (zero from n
+// to M/2; the zeros of the upper half are implied, their registers not read) at PM's forward first-pass input positions on entry and the result
 // at PM's inverse last-pass output positions on exit.  The chirp's spectrum
 // is loaded after the forward transform's last pass; `hook` runs after the
 // inverse's (loads issued before the last exchange take registers from its
@@ -72,7 +60,7 @@ __device__ __forceinline__ void blue_conv(cf (&v)[PM::E], const Buf &tw, int t, 
     const Elems<PM, -1, PM::np - 1> mid{t, PM::n};
     cf hv[PM::E];
     auto load_h = [&] { mid.all([&](int s, int o) { hv[s] = b.tab.get<cf>(8u * t, h + 8u * o); }); };
-    compute<PM, -1, 0>(v, tw, t);
+    compute_half<PM, -1>(v, t);
     Slots<PM> sl;
     passes_from<PM, -1, 1, false, false>(v, tw, t, L, sl, load_h);
     mid.all([&](int s, int) { v[s] = cmul(v[s], hv[s]); });
@@ -103,8 +91,12 @@ __device__ __forceinline__ void blue_fft(cf (&v)[PM::E], const Buf &tw, int t, c
     dst(v, out);
 }
 
-// transform DA, mid on its outputs, transform DB, callbacks as line_pair
-template <class PM, int DA, int DB, class Lds, class Src, class Pre, class Mid, class Dst>
+// transform DA, mid on its outputs, transform DB, callbacks as line_pair.
+// PHASELESS: mid scales each element by a real factor that depends on its
+// modulus alone (the modulus projection) and returns 0 past the end of the
+// line; the output chirp of DA and the input chirp of DB, conjugates of
+// modulus 1, then cancel and neither is applied.
+template <class PM, int DA, int DB, bool PHASELESS, class Lds, class Src, class Pre, class Mid, class Dst>
 __device__ __forceinline__ void blue_pair(cf (&v)[PM::E], const Buf &tw, int t, const Lds &L,
                                           const Blue &b, Src &src, Pre &pre, Mid &mid, Dst &dst)
 {
@@ -119,14 +111,13 @@ __device__ __forceinline__ void blue_pair(cf (&v)[PM::E], const Buf &tw, int t, 
     issue_loads();
     blue_apply_chirp<PM, DA>(v, ch, in);
     auto at_mid = [&] {
-        blue_load_chirp<PM>(ch, b, out);
+        if constexpr (!PHASELESS) blue_load_chirp<PM>(ch, b, out);
         pre(out);
     };
     blue_conv<PM, DA>(v, tw, t, L, b, at_mid);
-    blue_apply_chirp<PM, DA>(v, ch, out);
+    if constexpr (!PHASELESS) blue_apply_chirp<PM, DA>(v, ch, out);
     mid(v, out);
-    blue_apply_chirp<PM, DB>(v, ch, out);
-    blue_pad<PM, BlueOut<PM>>(v);
+    if constexpr (!PHASELESS) blue_apply_chirp<PM, DB>(v, ch, out);
     auto at_end = [&] { blue_load_chirp<PM>(ch, b, out); };
     blue_conv<PM, DB>(v, tw, t, L, b, at_end);
     blue_apply_chirp<PM, DB>(v, ch, out);
@@ -143,11 +134,11 @@ __device__ __forceinline__ void xfft(cf (&v)[P::E], const Buf &tw, int t, const 
     else line_fft<P, DIR>(v, tw, t, L, src, pre, dst);
 }
 
-template <class P, int DA, int DB, bool BL, int WHEN, class Lds, class Src, class Pre, class Mid, class Dst>
+template <class P, int DA, int DB, bool BL, int WHEN, bool PHASELESS, class Lds, class Src, class Pre, class Mid, class Dst>
 __device__ __forceinline__ void xpair(cf (&v)[P::E], const Buf &tw, int t, const Lds &L, const Blue &b,
                                       Src &src, Pre &pre, Mid &mid, Dst &dst)
 {
-    if constexpr (BL) blue_pair<P, DA, DB>(v, tw, t, L, b, src, pre, mid, dst);
+    if constexpr (BL) blue_pair<P, DA, DB, PHASELESS>(v, tw, t, L, b, src, pre, mid, dst);
     else line_pair<P, DA, DB, WHEN>(v, tw, t, L, src, pre, mid, dst);
 }
 

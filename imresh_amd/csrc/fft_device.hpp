@@ -130,6 +130,17 @@ __device__ __forceinline__ void bf4io(cf a, cf b, cf c, cf d, cf &o0, cf &o1, cf
     o3 = csub(t1, t3);
 }
 
+// the same for c = d = 0
+template <int DIR>
+__device__ __forceinline__ void bf4io_half(cf a, cf b, cf &o0, cf &o1, cf &o2, cf &o3)
+{
+    const cf t3 = rot<DIR>(b);
+    o0 = cadd(a, b);
+    o2 = csub(a, b);
+    o1 = cadd(a, t3);
+    o3 = csub(a, t3);
+}
+
 template <int DIR>
 __device__ __forceinline__ void bf4(cf *v)
 {
@@ -138,13 +149,19 @@ __device__ __forceinline__ void bf4(cf *v)
     v[0] = o0; v[1] = o1; v[2] = o2; v[3] = o3;
 }
 
-template <int DIR>
+// HALF: the upper half of the inputs is 0 and is not read
+template <int DIR, bool HALF = false>
 __device__ __forceinline__ void bf8(cf *v)
 {
     constexpr float c = 0.707106781f;
     cf e0, e1, e2, e3, o0, o1, o2, o3;
-    bf4io<DIR>(v[0], v[2], v[4], v[6], e0, e1, e2, e3);
-    bf4io<DIR>(v[1], v[3], v[5], v[7], o0, o1, o2, o3);
+    if constexpr (HALF) {
+        bf4io_half<DIR>(v[0], v[2], e0, e1, e2, e3);
+        bf4io_half<DIR>(v[1], v[3], o0, o1, o2, o3);
+    } else {
+        bf4io<DIR>(v[0], v[2], v[4], v[6], e0, e1, e2, e3);
+        bf4io<DIR>(v[1], v[3], v[5], v[7], o0, o1, o2, o3);
+    }
     o1 = cmul(o1, mkc(c, DIR * c));
     o2 = rot<DIR>(o2);
     o3 = cmul(o3, mkc(-c, DIR * c));
@@ -154,15 +171,19 @@ __device__ __forceinline__ void bf8(cf *v)
     v[3] = cadd(e3, o3); v[7] = csub(e3, o3);
 }
 
-template <int DIR>
+template <int DIR, bool HALF = false>
 __device__ __forceinline__ void bf16(cf *v)
 {
     constexpr float c1 = 0.923879533f, s1 = 0.382683432f, c2 = 0.707106781f;
     cf y[16];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-        bf4io<DIR>(v[q], v[q + 4], v[q + 8], v[q + 12], y[4 * q + 0], y[4 * q + 1], y[4 * q + 2],
-                   y[4 * q + 3]);
+    for (int q = 0; q < 4; ++q) {
+        if constexpr (HALF)
+            bf4io_half<DIR>(v[q], v[q + 4], y[4 * q + 0], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]);
+        else
+            bf4io<DIR>(v[q], v[q + 4], v[q + 8], v[q + 12], y[4 * q + 0], y[4 * q + 1], y[4 * q + 2],
+                       y[4 * q + 3]);
+    }
     // y[4*q + s] *= W16^(q*s), W16^k = (cos(2 pi k/16), DIR sin(2 pi k/16))
     y[5] = cmul(y[5], mkc(c1, DIR * s1));     // k = 1
     y[6] = cmul(y[6], mkc(c2, DIR * c2));     // k = 2
@@ -413,6 +434,22 @@ __device__ __forceinline__ void compute_tw(cf (&v)[P::E], const TwRegs<P, DIR, I
                     v[b * Q::R + r] = twmul<DIR>(v[b * Q::R + r], w.w[b * (Q::R - 1) + r - 1]);
             }
             bfly<Q::R, DIR>(&v[b * Q::R]);
+        }
+    }
+}
+
+// the first pass of a line whose upper half is 0 (and whose registers there
+// are not read)
+template <class P, int DIR>
+__device__ __forceinline__ void compute_half(cf (&v)[P::E], int t)
+{
+    using Q = PassOf<P, DIR, 0>;
+    static_assert(Q::R == 8 || Q::R == 16, "first radix of a convolution plan");
+#pragma unroll
+    for (int b = 0; b < Q::B; ++b) {
+        if (Q::full() || t + b * Q::T < Q::nb) {
+            if constexpr (Q::R == 8) bf8<DIR, true>(&v[b * Q::R]);
+            else bf16<DIR, true>(&v[b * Q::R]);
         }
     }
 }

@@ -106,14 +106,14 @@ __global__ void __launch_bounds__(C *P::T, 4) k_col(ColArgs a)
         const Buf X(a.X + wb, 8 * left);
         const Buf M(a.M + mb, 4 * ((size_t) (n - 1) * MP + W - (size_t) bid * C));
         const unsigned m0 = ((unsigned) (t * MP) + c0) * 4u | out_of;
-        float m[P::E];
+        float m[P::E] = {};   // 0 past the end of a line
         auto g0 = ld(X);
         auto pre = [&](const auto &el) {
             el.load([&](int s, int o) { m[s] = M.get<float>(m0, 4u * (unsigned) o * (unsigned) MP); });
         };
         auto mid = [&](auto &x, const auto &el) { modulus_project_line<P::E>(x, m, el); };
         auto sl = st(X);
-        xpair<P, -1, +1, BL, WHEN>(v, tw, t, L, bl, g0, pre, mid, sl);
+        xpair<P, -1, +1, BL, WHEN, true>(v, tw, t, L, bl, g0, pre, mid, sl);
     }
 }
 

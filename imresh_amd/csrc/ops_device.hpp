@@ -53,19 +53,20 @@ template <int E, class El>
 __device__ __forceinline__ void modulus_project_line(cf (&v)[E], const float (&m)[E], const El &el)
 {
     float low = 1e-30f;
-    el.load([&](int s, int o) {
+    el.all([&](int s, int o) {
         const float n2 = v[s].x * v[s].x + v[s].y * v[s].y;
         if (el.inside(o)) low = fminf(low, n2);
     });
     if (low >= 1e-30f) {
-        // (elements past the end of a line are 0 and have to stay finite)
-        el.load([&](int s, int) {
+        // (elements past the end of a line have modulus 0: they become 0 if
+        // the reciprocal root stays finite)
+        el.all([&](int s, int) {
             float n2 = v[s].x * v[s].x + v[s].y * v[s].y;
             if constexpr (El::span < El::Q::nb * El::Q::R) n2 = fmaxf(n2, 1e-30f);
             v[s] = modulus_project_fast(v[s], n2, m[s]);
         });
     } else {
-        el.load([&](int s, int) {
+        el.all([&](int s, int) {
             const float n2 = v[s].x * v[s].x + v[s].y * v[s].y;
             v[s] = n2 >= 1e-30f ? modulus_project_fast(v[s], n2, m[s]) : modulus_project(v[s], m[s]);
         });

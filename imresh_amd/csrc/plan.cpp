@@ -361,7 +361,7 @@ int launch_col_fourstep(const Plan2D &p, ColArgs a, hipStream_t s)
     Plan2D q = p;
     q.H = h2;
     IMR_CHECK(get_line_plan(dev, h2, &q.col));
-    q.colVar = col_variants(q.col) / 3 * 2;   // the plan's tile, modulus read early
+    q.colVar = 0;   // the plan's tile, modulus read at the junction
     ColArgs b = a;
     b.batch = images;
     b.sub = 8;
