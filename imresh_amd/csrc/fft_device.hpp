@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "plans.hpp"
 
 namespace imr {
 
@@ -405,15 +406,16 @@ __device__ __forceinline__ void load_tw(TwRegs<P, DIR, I> &w, const Buf &tw, int
         for (int b = 0; b < Q::B; ++b) {
             const int j = t + b * Q::T;
             if (Q::full() || j < Q::nb) {
-                const unsigned k = (unsigned) (j % Q::NS) * (8u * (Q::R - 1));
+                const unsigned k = (unsigned) (j % Q::NS);
 #pragma unroll
                 for (int r = 1; r + 1 < Q::R; r += 2) {
-                    const cf2 x = tw.get<cf2>(k + 8u * (r - 1), 8u * Q::TWOFF);
+                    const cf2 x = tw.get<cf2>(16u * k, 8u * (Q::TWOFF + tw_index(Q::R, Q::NS, 0, r)));
                     w.w[b * (Q::R - 1) + r - 1] = mkc(x.x, x.y);
                     w.w[b * (Q::R - 1) + r] = mkc(x.z, x.w);
                 }
                 if constexpr ((Q::R & 1) == 0)
-                    w.w[b * (Q::R - 1) + Q::R - 2] = tw.get<cf>(k + 8u * (Q::R - 2), 8u * Q::TWOFF);
+                    w.w[b * (Q::R - 1) + Q::R - 2] =
+                        tw.get<cf>(8u * k, 8u * (Q::TWOFF + tw_index(Q::R, Q::NS, 0, Q::R - 1)));
             }
         }
     }

@@ -54,15 +54,17 @@ const PlanInfo *find_info(int n)
 }
 
 // exp(-2 pi i r k / (ns R)) for every pass of a radix sequence, evaluated in
-// double; layout as Plan::twoff (k-major, r = 1..R-1)
+// double; one pass after the other (Plan::twoff), each laid out by tw_index
 void append_twiddles(const std::vector<int> &rad, std::vector<float2> &tw)
 {
     int ns = 1;
     for (int R : rad) {
+        const size_t base = tw.size();
+        tw.resize(base + (size_t) ns * (R - 1));
         for (int k = 0; k < ns; ++k)
             for (int r = 1; r < R; ++r) {
                 const double a = -2.0 * M_PI * (double) r * (double) k / ((double) ns * R);
-                tw.push_back(make_float2((float) std::cos(a), (float) std::sin(a)));
+                tw[base + tw_index(R, ns, k, r)] = make_float2((float) std::cos(a), (float) std::sin(a));
             }
         ns *= R;
     }

@@ -30,6 +30,16 @@ constexpr int kRowThreadsTarget = 256;   // row workgroup size target
 constexpr int kColMaxCols = 8;           // columns per column workgroup (64 B per row)
 constexpr int kLdsBudget = 144 * 1024;   // dynamic LDS per workgroup (of 160 KiB)
 
+// place of exp(-2 pi i r k / (ns R)), 1 <= r < R, among its pass's ns*(R-1)
+// twiddles: the pairs r = (1, 2), (3, 4), ... one after the other, each with
+// its k consecutive, and a single last r (R even) after them.  Threads of
+// consecutive k then load a pair as 16 consecutive bytes each.
+__host__ __device__ constexpr int tw_index(int R, int ns, int k, int r)
+{
+    const int q = (r - 1) / 2;
+    return r == R - 1 && R % 2 == 0 ? 2 * q * ns + k : 2 * (q * ns + k) + (r - 1) % 2;
+}
+
 // E: complex values per thread and pass (the thread count per line follows)
 template <int E_, int N, int... Rs>
 struct PlanE {
