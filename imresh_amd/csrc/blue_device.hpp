@@ -13,6 +13,8 @@
 //   tab[0, M/2)         a_j, zero from n on (2n - 1 <= M: n <= M/2)
 //   tab[M/2, 3M/2)      FFT_M(wrap(conj a)) / M   (forward transform)
 //   tab[3M/2, 5M/2)     FFT_M(wrap(a)) / M        (inverse transform)
+// each in the order of the registers that read it (blue_index): the chirp by
+// PM's forward first pass, the spectra by its forward last one.
 // wrap(b)[m] = b_m for m < n, b_(M-m) for m > M-n, 0 otherwise.
 #pragma once
 
@@ -31,19 +33,38 @@ struct Blue {
 template <class PM> using BlueIn = Elems<PM, -1, 0, true>;
 template <class PM> using BlueOut = Elems<PM, +1, PM::np - 1, true>;
 
-// chirp a_(t+o) of a thread's elements
-template <class PM, class El>
-__device__ __forceinline__ void blue_load_chirp(cf (&ch)[PM::E], const Blue &b, const El &el)
+// a thread's `count` values of a table at byte `base`, in pairs
+template <class PM, int count>
+__device__ __forceinline__ void blue_load(cf (&x)[count], const Blue &b, int t, unsigned base)
 {
-    el.all([&](int s, int o) { ch[s] = b.tab.get<cf>(8u * el.t, 8u * o); });
+    static_assert(count % 2 == 0 && PM::E % 2 == 0, "values load in pairs");
+#pragma unroll
+    for (int q = 0; q < count; q += 2) {
+        const cf2 p = b.tab.get<cf2>(16u * t, base + 8u * blue_index(q, 0, PM::T));
+        x[q] = mkc(p.x, p.y);
+        x[q + 1] = mkc(p.z, p.w);
+    }
 }
+
+// chirp a_(t+o) of a thread's elements below M/2: register s = b*R + r has
+// value b*R/2 + r
+template <class PM>
+struct Chirp {
+    cf a[PM::E / 2];
+    __device__ __forceinline__ void load(const Blue &b, int t) { blue_load<PM, PM::E / 2>(a, b, t, 0u); }
+    __device__ __forceinline__ cf at(int s) const
+    {
+        constexpr int R = PM::rf[0];
+        return a[s / R * (R / 2) + s % R];
+    }
+};
 
 // v <- chirped line (conjugated chirp for the inverse): the table's zeros
 // clear what lies past its end
 template <class PM, int DIR, class El>
-__device__ __forceinline__ void blue_apply_chirp(cf (&v)[PM::E], const cf (&ch)[PM::E], const El &el)
+__device__ __forceinline__ void blue_apply_chirp(cf (&v)[PM::E], const Chirp<PM> &ch, const El &el)
 {
-    el.all([&](int s, int) { v[s] = cmul(v[s], DIR < 0 ? ch[s] : mkc(ch[s].x, -ch[s].y)); });
+    el.all([&](int s, int) { v[s] = cmul(v[s], DIR < 0 ? ch.at(s) : mkc(ch.at(s).x, -ch.at(s).y)); });
 }
 
 // circular convolution with the chirp: v holds the chirped line (zero from n
@@ -57,13 +78,14 @@ __device__ __forceinline__ void blue_conv(cf (&v)[PM::E], const Buf &tw, int t, 
                                           const Blue &b, Hook &hook)
 {
     constexpr unsigned h = 8u * (PM::n / 2 + (DIR < 0 ? 0 : PM::n));
-    const Elems<PM, -1, PM::np - 1> mid{t, PM::n};
+    static_assert(PM::T * PM::E == PM::n, "every register of every thread is an element");
     cf hv[PM::E];
-    auto load_h = [&] { mid.all([&](int s, int o) { hv[s] = b.tab.get<cf>(8u * t, h + 8u * o); }); };
+    auto load_h = [&] { blue_load<PM, PM::E>(hv, b, t, h); };
     compute_half<PM, -1>(v, t);
     Slots<PM> sl;
     passes_from<PM, -1, 1, false, false>(v, tw, t, L, sl, load_h);
-    mid.all([&](int s, int) { v[s] = cmul(v[s], hv[s]); });
+#pragma unroll
+    for (int s = 0; s < PM::E; ++s) v[s] = cmul(v[s], hv[s]);
     compute<PM, +1, 0>(v, tw, t);
     passes_from<PM, +1, 1, true, false>(v, tw, t, L, sl, hook);
 }
@@ -75,15 +97,15 @@ __device__ __forceinline__ void blue_fft(cf (&v)[PM::E], const Buf &tw, int t, c
 {
     const BlueIn<PM> in{t, b.n};
     const BlueOut<PM> out{t, b.n};
-    cf ch[PM::E];
+    Chirp<PM> ch;
 #pragma unroll
     for (int s = 0; s < PM::E; ++s) v[s] = mkc(0.f, 0.f);
     src(v, in);
-    blue_load_chirp<PM>(ch, b, in);
+    ch.load(b, t);
     issue_loads();
     blue_apply_chirp<PM, DIR>(v, ch, in);
     auto hook = [&] {
-        blue_load_chirp<PM>(ch, b, out);
+        ch.load(b, t);
         pre(out);
     };
     blue_conv<PM, DIR>(v, tw, t, L, b, hook);
@@ -103,22 +125,22 @@ __device__ __forceinline__ void blue_pair(cf (&v)[PM::E], const Buf &tw, int t, 
     static_assert(DA == -DB, "a pair runs opposite directions");
     const BlueIn<PM> in{t, b.n};
     const BlueOut<PM> out{t, b.n};
-    cf ch[PM::E];
+    Chirp<PM> ch;
 #pragma unroll
     for (int s = 0; s < PM::E; ++s) v[s] = mkc(0.f, 0.f);
     src(v, in);
-    blue_load_chirp<PM>(ch, b, in);
+    ch.load(b, t);
     issue_loads();
     blue_apply_chirp<PM, DA>(v, ch, in);
     auto at_mid = [&] {
-        if constexpr (!PHASELESS) blue_load_chirp<PM>(ch, b, out);
+        if constexpr (!PHASELESS) ch.load(b, t);
         pre(out);
     };
     blue_conv<PM, DA>(v, tw, t, L, b, at_mid);
     if constexpr (!PHASELESS) blue_apply_chirp<PM, DA>(v, ch, out);
     mid(v, out);
     if constexpr (!PHASELESS) blue_apply_chirp<PM, DB>(v, ch, out);
-    auto at_end = [&] { blue_load_chirp<PM>(ch, b, out); };
+    auto at_end = [&] { ch.load(b, t); };
     blue_conv<PM, DB>(v, tw, t, L, b, at_end);
     blue_apply_chirp<PM, DB>(v, ch, out);
     dst(v, out);

@@ -121,9 +121,11 @@ int blue_m(int n)
     return find_info(m) != nullptr ? m : 0;
 }
 
-// Bluestein tables of length n (layout in blue_device.hpp), float from double
-std::vector<float2> blue_tables(int n, int m)
+// Bluestein tables of length n for the convolution plan `pi` of length m
+// (layout in blue_device.hpp), float from double
+std::vector<float2> blue_tables(int n, const PlanInfo &pi)
 {
+    const int m = pi.n;
     std::vector<std::complex<double>> a(n), bf(m, 0.0), bi(m, 0.0);
     for (int j = 0; j < n; ++j) {
         // j^2 mod 2n keeps the angle exact for large j
@@ -141,12 +143,25 @@ std::vector<float2> blue_tables(int n, int m)
     }
     dft_any(bf);
     dft_any(bi);
+    // register s = b*R + r of thread t holds element t + b*T + r*m/R of a pass
+    // of radix R; registers 2q and 2q+1 of a thread lie together, the threads
+    // of a pair one after the other
+    auto lay = [&](int R, int used, auto value, std::vector<float2> &out) {
+        const size_t base = out.size();
+        const int B = m / R / pi.T;
+        out.resize(base + (size_t) B * used * pi.T);
+        for (int b = 0; b < B; ++b)
+            for (int r = 0; r < used; ++r)
+                for (int t = 0; t < pi.T; ++t) {
+                    const std::complex<double> x = value(t + b * pi.T + r * (m / R));
+                    out[base + blue_index(b * used + r, t, pi.T)] = make_float2((float) x.real(), (float) x.imag());
+                }
+    };
+    const int first = pi.rad[0], last = pi.rad[pi.np - 1];
     std::vector<float2> out;
-    out.reserve((size_t) m / 2 + 2 * m);
-    for (int j = 0; j < n; ++j) out.push_back(make_float2((float) a[j].real(), (float) a[j].imag()));
-    out.resize((size_t) m / 2, make_float2(0.f, 0.f));
-    for (int k = 0; k < m; ++k) out.push_back(make_float2((float) (bf[k].real() / m), (float) (bf[k].imag() / m)));
-    for (int k = 0; k < m; ++k) out.push_back(make_float2((float) (bi[k].real() / m), (float) (bi[k].imag() / m)));
+    lay(first, first / 2, [&](int e) { return e < n ? a[e] : std::complex<double>(0.0); }, out);
+    lay(last, last, [&](int e) { return bf[e] / (double) m; }, out);
+    lay(last, last, [&](int e) { return bi[e] / (double) m; }, out);
     return out;
 }
 
@@ -195,7 +210,7 @@ int get_line_plan(int device, int n, LinePlan *out)
         LinePlan lm;
         IMR_CHECK(get_line_plan(device, m, &lm));
         float2 *dev = nullptr;
-        IMR_CHECK(upload_table(device, blue_tables(n, m), &dev));
+        IMR_CHECK(upload_table(device, blue_tables(n, *find_info(m)), &dev));
         LinePlan lp = lm;
         lp.n = n;
         lp.blue = 1;

@@ -40,6 +40,10 @@ __host__ __device__ constexpr int tw_index(int R, int ns, int k, int r)
     return r == R - 1 && R % 2 == 0 ? 2 * q * ns + k : 2 * (q * ns + k) + (r - 1) % 2;
 }
 
+// place of a thread's q-th value in a Bluestein table of T threads a line:
+// values 2i and 2i+1 of a thread together, the threads one after the other
+__host__ __device__ constexpr int blue_index(int q, int t, int T) { return 2 * (q / 2 * T + t) + q % 2; }
+
 // E: complex values per thread and pass (the thread count per line follows)
 template <int E_, int N, int... Rs>
 struct PlanE {
