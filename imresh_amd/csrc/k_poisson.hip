@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(256) k_poisson_modulus(float *m, size_t n, con
          i += (size_t) gridDim.x * blockDim.x) {
         const double v = (double) m[i];
         const double lam = t > 0.0 ? photons * (v * v) / t : 0.0;
-        m[i] = (float) pois::sqrt_d(pois::poisson(lam, seed, (uint64_t) i));
+        m[i] = pois::sqrt_count(pois::poisson(lam, seed, (uint64_t) i));
     }
 }
 

@@ -96,6 +96,49 @@ __host__ __device__ inline double sqrt_d(double x)
     return s;
 }
 
+// (float) sqrt_d(k) of an integer-valued k >= 0.  Below 2^24 the correctly
+// rounded single-precision root is the same: k is exact in float, and
+// sqrt(k) is never within 2^-50 (relative) of the midpoint of two floats,
+// whose square would differ from k by less than its last bit.
+__host__ __device__ inline float sqrt_count(double k)
+{
+    return k < 16777216.0 ? sqrtf((float) k) : (float) sqrt_d(k);
+}
+
+// 1/k for the small integers, as a double and the double nearest to what it
+// leaves out (|lo| < 2^-53 hi)
+struct Reciprocals {
+    static constexpr int kCount = 64;
+    double hi[kCount + 1], lo[kCount + 1];
+    constexpr Reciprocals() : hi(), lo()
+    {
+        for (int k = 1; k <= kCount; ++k) {
+            int e = 52;   // 2^e / k in [2^52, 2^53)
+            unsigned __int128 num = (unsigned __int128) 1 << 52;
+            while (num / (unsigned) k < ((unsigned __int128) 1 << 52)) {
+                num <<= 1;
+                ++e;
+            }
+            const unsigned __int128 q = (num + (unsigned) k / 2) / (unsigned) k;
+            const long long rem = (long long) (__int128) (num - q * (unsigned) k);
+            double scale = 1.0;
+            for (int i = 0; i < e; ++i) scale *= 0.5;
+            hi[k] = (double) (unsigned long long) q * scale;
+            lo[k] = (double) rem / (double) k * scale;
+        }
+    }
+};
+
+// x / k, correctly rounded as the division is, for 1 <= k <= kCount and x >= 0
+// far from underflow: x*hi + x*lo is exact to 2^-104, a quotient by k keeps
+// 2^-60 from every rounding boundary and is never on one (k times an odd
+// 54-bit number has more than 53 bits).
+__host__ __device__ inline double div_small(double x, int k, const Reciprocals &r)
+{
+    const double q = x * r.hi[k];
+    return q + __builtin_fma(x, r.lo[k], __builtin_fma(x, r.hi[k], -q));
+}
+
 // log k! for an integer-valued k >= 0
 __host__ __device__ inline double log_factorial(double k)
 {
@@ -148,7 +191,15 @@ __host__ __device__ inline double poisson(double lam, uint64_t seed, uint64_t id
         double u, unused;
         uniforms(seed, idx, 0u, &u, &unused);
         double p = exp_d(-lam), F = p, k = 0.0;
-        for (int i = 0; i < 1000 && u > F; ++i) {
+        int i = 0;
+        // the step number is uniform in a wave: its reciprocal is a scalar load
+        static constexpr Reciprocals recip;
+        for (; i < Reciprocals::kCount && u > F; ++i) {
+            k = k + 1.0;
+            p = div_small(p * lam, i + 1, recip);
+            F = F + p;
+        }
+        for (; i < 1000 && u > F; ++i) {
             k = k + 1.0;
             p = p * lam / k;
             F = F + p;
@@ -156,12 +207,10 @@ __host__ __device__ inline double poisson(double lam, uint64_t seed, uint64_t id
         return k;
     }
     const double slam = sqrt_d(lam);
-    const double loglam = log_d(lam);
     const double b = 0.931 + 2.53 * slam;
     const double a = -0.059 + 0.02483 * b;
     const double invalpha = 1.1239 + 1.1328 / (b - 3.4);
     const double vr = 0.9277 - 3.6224 / (b - 2.0);
-    const double log_invalpha = log_d(invalpha);
     for (uint32_t it = 0; it < 256u; ++it) {
         double u1, v;
         uniforms(seed, idx, it, &u1, &v);
@@ -171,8 +220,9 @@ __host__ __device__ inline double poisson(double lam, uint64_t seed, uint64_t id
         const double k = floor((2.0 * a / us + b) * U + lam + 0.43);
         if (us >= 0.07 && v <= vr) return k;
         if (k < 0.0 || (us < 0.013 && v > us)) continue;
-        const double lhs = log_d(v) + log_invalpha - log_d(a / (us * us) + b);
-        const double rhs = -lam + k * loglam - log_factorial(k);
+        // (the logarithms only where the squeeze above has not decided)
+        const double lhs = log_d(v) + log_d(invalpha) - log_d(a / (us * us) + b);
+        const double rhs = -lam + k * log_d(lam) - log_factorial(k);
         if (lhs <= rhs) return k;
     }
     return floor(lam + 0.5);
