@@ -20,8 +20,20 @@ __global__ void __launch_bounds__(kSumThreads) k_sq_sum(const float *m, size_t n
 {
     __shared__ double s[kSumThreads];
     const size_t lanes = (size_t) kPoissonSumBlocks * kSumThreads;
+    // the adds of a lane are one chain in a fixed order; its loads go kAhead at
+    // a time (one by one, the loop was a chain of memory round trips: 18 us
+    // for 2048^2 of its 148 us simulation, which takes 135 us like this)
+    constexpr int kAhead = 16;
     double acc = 0.0;
-    for (size_t i = blockIdx.x * (size_t) kSumThreads + threadIdx.x; i < n; i += lanes) {
+    size_t i = blockIdx.x * (size_t) kSumThreads + threadIdx.x;
+    for (; i + (kAhead - 1) * lanes < n; i += kAhead * lanes) {
+        float v[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) v[k] = m[i + k * lanes];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) acc = acc + (double) v[k] * (double) v[k];
+    }
+    for (; i < n; i += lanes) {
         const double v = (double) m[i];
         acc = acc + v * v;
     }
