@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(C *P::T, 4) k_col(ColArgs a)
         };
         auto mid = [&](auto &x, const auto &el) { modulus_project_line<P::E>(x, m, el); };
         auto sl = st(X);
-        xpair<P, -1, +1, BL, WHEN, true>(v, tw, t, L, bl, g0, pre, mid, sl);
+        xpair<P, -1, +1, BL, WHEN>(v, tw, t, L, bl, g0, pre, mid, sl);
     }
 }
 

@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
             el.load([&](int s, int) { x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta); });
             if (valid) el.store([&](int s, int o) { G.put(x[s], 8 * e0, 8 * o); });
         };
-        xpair<P, +1, -1, BL, WHEN, false>(v, tw, t, L, bl, ldX, pre, mid, stX);
+        xpair<P, +1, -1, BL, WHEN>(v, tw, t, L, bl, ldX, pre, mid, stX);
     }
 }
 
