@@ -227,7 +227,7 @@ int ws_checkout(int device, int W, int H, hipStream_t s, Workspace **out)
     // a busy workspace taken over (kMaxWorkspaces of this size in use): its
     // previous user's work runs first.  Should that work not finish in
     // reasonable time (a caller stream destroyed with its work dropped would
-    // never run the host function), the workspace stays in the pool and a
+    // never run the kernel that marks it idle), the workspace stays in the pool and a
     // new one is allocated instead of waiting on.
     (void) s;
     if (!ws_wait_idle(w, 10.0)) {
@@ -383,8 +383,8 @@ namespace {
 
 // ---------------------------------------------------------------- autotuner
 // Picks, per device and image size, the fastest row-pass and column-pass
-// kernel variant (element budget / rows or columns per workgroup / LDS
-// exchange) by timing each on a synthetic resident state with HIP events, the
+// kernel variant (where the junction's operands are read / rows or columns per
+// workgroup) by timing each on a synthetic resident state with HIP events, the
 // row and the column pass in turn as an iteration runs them: alone, a pass of
 // 4096^2 finds its planes in the Infinity Cache, which the other pass leaves
 // only in part (column pass 115 us alone, 162 us in turn).

@@ -25,7 +25,7 @@ def main() -> int:
     ap.add_argument("--size", type=int, default=2048)
     ap.add_argument("--reps", type=int, default=8)
     ap.add_argument("--variants", default="",
-                    help="row,column kernel variants to pin instead of autotuning (e.g. 0,5)")
+                    help="row,column kernel variants to pin instead of autotuning (e.g. 1,0)")
     a = ap.parse_args()
     L = im.lib()
     nbytes = 128 << 20
