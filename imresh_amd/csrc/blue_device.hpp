@@ -59,12 +59,17 @@ struct Chirp {
     }
 };
 
-// v <- chirped line (conjugated chirp for the inverse): the table's zeros
-// clear what lies past its end
-template <class PM, int DIR, class El>
+// v <- chirped line (conjugated chirp for the inverse).  What lies past the
+// line's end becomes 0 by the table's zeros if it is finite; CLEAR sets it to
+// 0 whatever it is (the first transform's values there, which may overflow
+// where the line does not)
+template <class PM, int DIR, bool CLEAR = false, class El>
 __device__ __forceinline__ void blue_apply_chirp(cf (&v)[PM::E], const Chirp<PM> &ch, const El &el)
 {
-    el.all([&](int s, int) { v[s] = cmul(v[s], DIR < 0 ? ch.at(s) : mkc(ch.at(s).x, -ch.at(s).y)); });
+    el.all([&](int s, int o) {
+        v[s] = cmul(v[s], DIR < 0 ? ch.at(s) : mkc(ch.at(s).x, -ch.at(s).y));
+        if (CLEAR && !el.inside(o)) v[s] = mkc(0.f, 0.f);
+    });
 }
 
 // circular convolution with the chirp: v holds the chirped line (zero from n
@@ -138,7 +143,7 @@ __device__ __forceinline__ void blue_pair(cf (&v)[PM::E], const Buf &tw, int t, 
     blue_conv<PM, DA>(v, tw, t, L, b, at_mid);
     blue_apply_chirp<PM, DA>(v, ch, out);
     mid(v, out);
-    blue_apply_chirp<PM, DB>(v, ch, out);
+    blue_apply_chirp<PM, DB, true>(v, ch, out);
     auto at_end = [&] { ch.load(b, t); };
     blue_conv<PM, DB>(v, tw, t, L, b, at_end);
     blue_apply_chirp<PM, DB>(v, ch, out);

@@ -48,7 +48,9 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
     const int n = BL ? a.len : P::n;
     const int l = threadIdx.x / T, t = threadIdx.x - l * T;
     // planes from the workgroup's first row to the image's last: loads of the
-    // rows past the end return 0
+    // rows past the end return 0, and so do those of lanes past the end of a
+    // Bluestein line (at), where the next row begins: another workgroup may be
+    // rewriting it, and a value that overflowed there must not come in
     const size_t wb = (size_t) b * a.istride + (size_t) blockIdx.x * NL * n;
     const size_t left = (size_t) (a.H - (int) blockIdx.x * NL) * n;
     const unsigned e0 = (unsigned) (l * n + t);
@@ -58,9 +60,10 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
     const Buf tw(a.tw, 8 * (size_t) (2 * P::n - 1));
     const LdsLine<1, 64 % T == 0> L{smem + l * lds_elems(P::n)};
     cf v[P::E];
+    auto at = [](unsigned e, const auto &el, int o) { return el.inside(o) ? e : kOutside; };
     auto ld = [&](const Buf &p) {
         return [&](auto &x, const auto &el) {
-            el.load([&](int s, int o) { x[s] = p.template get<cf>(8 * e0, 8 * o); });
+            el.load([&](int s, int o) { x[s] = p.template get<cf>(at(8 * e0, el, o), 8 * o); });
         };
     };
     auto st = [&](const Buf &p) {
@@ -96,7 +99,7 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
         auto ldX = ld(X);
         auto pre = [&](const auto &el) {
             if constexpr ((fl & kRowError) != 0)
-                el.load([&](int s, int o) { m[s] = mask.get<uint8_t>(e0, o); });
+                el.load([&](int s, int o) { m[s] = mask.get<uint8_t>(at(e0, el, o), o); });
         };
         auto sl = [&](auto &x, const auto &el) {
             if (!valid) return;
@@ -134,10 +137,10 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
             float bv[P::E];
             uint8_t m[P::E];
             el.load([&](int s, int o) {
-                x[s] = X.get<cf>(8 * e0, 8 * o);
-                g[s] = G.get<cf>(8 * e0, 8 * o);
-                if constexpr (cut) bv[s] = B2.get<float>(4 * e0, 4 * o);
-                else m[s] = mask.get<uint8_t>(e0, o);
+                x[s] = X.get<cf>(at(8 * e0, el, o), 8 * o);
+                g[s] = G.get<cf>(at(8 * e0, el, o), 8 * o);
+                if constexpr (cut) bv[s] = B2.get<float>(at(4 * e0, el, o), 4 * o);
+                else m[s] = mask.get<uint8_t>(at(e0, el, o), o);
             });
             el.load([&](int s, int) {
                 if constexpr (cut) m[s] = bv[s] < thr ? 1 : 0;
@@ -157,8 +160,8 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
         auto ldX = ld(X);
         auto pre = [&](const auto &el) {
             el.load([&](int s, int o) {
-                g[s] = G.get<cf>(8 * e0, 8 * o);
-                m[s] = mask.get<uint8_t>(e0, o);
+                g[s] = G.get<cf>(at(8 * e0, el, o), 8 * o);
+                m[s] = mask.get<uint8_t>(at(e0, el, o), o);
             });
         };
         auto mid = [&](auto &x, const auto &el) {
