@@ -73,6 +73,11 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
     };
     auto none = [](const auto &) {};
     auto stX = st(X);
+    // The constraint runs over initialised operands and every element: over
+    // operands that only el.load's branches set, in branches of its own, the
+    // compiler kept all of it live at once (Bluestein RK_FIRST of 64- and
+    // 512-point convolutions: 1849 and 1293 spilled registers; a 250^2
+    // reconstruction of 4 cycles 332 us, 252 us like this)
 
     if constexpr (K == RK_FWD || K == RK_INV || K == RK_FWD_NORM) {
         const Buf in(a.in + wb, 8 * left);
@@ -133,16 +138,16 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
         const Buf B2(a.B2 + wb, 4 * left);
         const float beta = a.beta;
         auto g0 = [&](auto &x, const auto &el) {
-            cf g[P::E];
-            float bv[P::E];
-            uint8_t m[P::E];
+            cf g[P::E] = {};
+            float bv[P::E] = {};
+            uint8_t m[P::E] = {};
             el.load([&](int s, int o) {
                 x[s] = X.get<cf>(at(8 * e0, el, o), 8 * o);
                 g[s] = G.get<cf>(at(8 * e0, el, o), 8 * o);
                 if constexpr (cut) bv[s] = B2.get<float>(at(4 * e0, el, o), 4 * o);
                 else m[s] = mask.get<uint8_t>(at(e0, el, o), o);
             });
-            el.load([&](int s, int) {
+            el.all([&](int s, int) {
                 if constexpr (cut) m[s] = bv[s] < thr ? 1 : 0;
                 x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta);
             });
@@ -155,8 +160,8 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
         xfft<P, -1, BL>(v, tw, t, L, bl, g0, none, stX);
     } else if constexpr (K == RK_MID) {
         const float beta = a.beta;
-        cf g[P::E];
-        uint8_t m[P::E];
+        cf g[P::E] = {};
+        uint8_t m[P::E] = {};
         auto ldX = ld(X);
         auto pre = [&](const auto &el) {
             el.load([&](int s, int o) {
@@ -165,7 +170,7 @@ __global__ void __launch_bounds__(NL *P::T, 4) k_row(RowArgs a)
             });
         };
         auto mid = [&](auto &x, const auto &el) {
-            el.load([&](int s, int) { x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta); });
+            el.all([&](int s, int) { x[s] = hio_constraint(g[s], x[s], m[s] == 1, beta); });
             if (valid) el.store([&](int s, int o) { G.put(x[s], 8 * e0, 8 * o); });
         };
         xpair<P, +1, -1, BL, WHEN>(v, tw, t, L, bl, ldX, pre, mid, stX);
