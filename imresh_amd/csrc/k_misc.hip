@@ -388,11 +388,20 @@ __global__ void k_store_words(float *dst, unsigned n, StoreWords a)
 }
 
 // Completion word of a pooled buffer: a value in coherent host memory, stored
-// behind the work that uses the buffer.  One thread, ~2 us on the stream; a
-// host function there held the stream until a host thread had woken and run
-// it (forward model and blur calls: see launch_signal).
+// behind the work that uses the buffer.  One thread; a host function there
+// held the stream until a host thread had woken and run it (operators of a
+// mask update on 1000x1200: 99 us; 63 us with the word and the reductions'
+// results stored straight into pinned memory).  REPLAYED:
+// captured in a caller's graph, where every replay comes here again, also
+// after the buffer has been handed on with a later value, which must stay
+// (the values of a buffer ascend; reading the word back is a round trip over
+// PCIe, so only captured calls do).
+template <bool REPLAYED>
 __global__ void k_signal(uint32_t *word, uint32_t value)
 {
+    if (REPLAYED &&
+        (int32_t) (value - __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) <= 0)
+        return;
     __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -409,7 +418,12 @@ __global__ void __launch_bounds__(128) k_stage_words(float *host, const float *d
 // ------------------------------------------------------------ launchers
 int launch_signal(uint32_t *word, uint32_t value, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_signal, dim3(1), dim3(1), 0, s, word, value);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void) hipGetLastError();
+    if (capture == hipStreamCaptureStatusNone)
+        hipLaunchKernelGGL(k_signal<false>, dim3(1), dim3(1), 0, s, word, value);
+    else
+        hipLaunchKernelGGL(k_signal<true>, dim3(1), dim3(1), 0, s, word, value);
     return imr::launch_status(__FILE__, __LINE__);
 }
 
