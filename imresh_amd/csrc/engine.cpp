@@ -443,8 +443,8 @@ int autotune(int device, int W, int H, hipStream_t s, Workspace *w)
     const char *force = std::getenv("IMRESH_VARIANTS");
     const char *off = std::getenv("IMRESH_AUTOTUNE");
     if (force != nullptr && std::sscanf(force, "%d,%d", &rv, &cv) == 2) {
-        rv = std::min(std::max(rv, 0), std::max(nr - 1, 0));
-        cv = std::min(std::max(cv, 0), std::max(nc - 1, 0));
+        rv = std::min(std::max(rv, 0), row_variant_numbers(p.row) - 1);
+        cv = std::min(std::max(cv, 0), col_variant_numbers(p.col) - 1);
     } else if (!(off != nullptr && off[0] == '0') && (nr > 1 || nc > 1)) {
         // every variant once per round, best of kTuneRounds rounds: timing
         // the variants one after the other would bias against the first
@@ -1691,8 +1691,8 @@ int imresh_variant_counts(uint32_t width, uint32_t height, int *row_variants_out
     IMR_CHECK(current_device(&dev));
     Plan2D p;
     IMR_CHECK(get_plan2d(dev, width, height, &p));
-    if (row_variants_out) *row_variants_out = std::max(row_variants(p.row), 1);
-    if (col_variants_out) *col_variants_out = std::max(col_variants(p.col), 1);
+    if (row_variants_out) *row_variants_out = row_variant_numbers(p.row);
+    if (col_variants_out) *col_variants_out = col_variant_numbers(p.col);
     return IMRESH_OK;
 }
 

@@ -159,8 +159,11 @@ struct Plan2D {
     int colVar;      // kernel variant of the column pass (autotuned)
 };
 
+// the kernels a length has, and the variant numbers that name them
 int row_variants(const LinePlan &lp);
 int col_variants(const LinePlan &lp);
+int row_variant_numbers(const LinePlan &lp);
+int col_variant_numbers(const LinePlan &lp);
 void set_tuned_variants(int device, int W, int H, int rowVar, int colVar);
 bool get_tuned_variants(int device, int W, int H, int *rowVar, int *colVar);
 

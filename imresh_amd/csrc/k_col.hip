@@ -195,6 +195,7 @@ int launch_col_variant(int var, int mode, ColArgs a, hipStream_t s)
         return IMRESH_ERR_UNSUPPORTED_SIZE;   // a convolution length only
     } else {
         constexpr int ns = col_shape_count<N, Rs...>();
+        var %= col_variant_count<N, Rs...>();
         if constexpr (ns > 1) {
             if (var % ns == 1) return launch_when<P, 4>(var / ns, mode, a, s);
         }

@@ -277,6 +277,7 @@ int launch_row_variant(int var, int mode, RowArgs a, hipStream_t s)
         return IMRESH_ERR_UNSUPPORTED_SIZE;   // a convolution length only
     } else {
         constexpr int ns = row_shape_count<N, Rs...>();
+        var %= row_variant_count<N, Rs...>();
         if constexpr (ns > 1) {
             if (var % ns == 1) return launch_when<P, small_group<N, Rs...>()>(var / ns, mode, a, s);
         }
@@ -292,6 +293,7 @@ int row_variant_rows(int var)
     using P = Plan<N, Rs...>;
     if (var == kBlueVariant) return blue_rows<P>();
     constexpr int ns = row_shape_count<N, Rs...>();
+    var %= row_variant_count<N, Rs...>();
     return var % ns == 1 ? small_group<N, Rs...>() : P::L;
 }
 

@@ -3,6 +3,7 @@
 // kernel dispatch by plan group, and the Gaussian weights / sigma schedule
 // of the reference (computed on the host exactly as the reference does, so
 // the device blur uses bit-identical weights).
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <map>
@@ -444,6 +445,19 @@ int col_variants(const LinePlan &lp)
     default: return 0;
     }
 }
+
+// Power-of-two lines from 1024 points once had more kernels than now.  Their
+// numbers stay accepted, for the programs that pin what an earlier
+// imresh_autotune reported; a number past the kernels there are names one of
+// them again (the launch takes it modulo their count).
+static int accepted_numbers(const LinePlan &lp, int kernels, int upto2048, int above)
+{
+    const bool pow2 = !lp.blue && lp.n >= 1024 && (lp.n & (lp.n - 1)) == 0;
+    return std::max(kernels, !pow2 ? 1 : lp.n <= 2048 ? upto2048 : above);
+}
+
+int row_variant_numbers(const LinePlan &lp) { return accepted_numbers(lp, row_variants(lp), 10, 8); }
+int col_variant_numbers(const LinePlan &lp) { return accepted_numbers(lp, col_variants(lp), 10, 4); }
 
 // calcGaussianKernel.cpp:42-91: radius ceil(2.884402748387961466*sigma - 0.5),
 // float weights a*exp(i^2*b) summed in double, each divided by the sum.

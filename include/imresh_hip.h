@@ -360,8 +360,9 @@ int imresh_fft_shift(void *data_dev, uint32_t nx, uint32_t ny, uint32_t element_
  * internally, cudaShrinkWrap.cu:226). */
 int imresh_autotune(uint32_t width, uint32_t height, void *stream, int *row_variant,
                     int *col_variant);
-/* Number of row- and column-pass kernel variants of W x H (every variant
- * computes the same bits; they differ in tiling and scheduling). */
+/* Row- and column-pass variant numbers of W x H: imresh_set_variants takes
+ * 0 ... count - 1 (every variant computes the same bits; they differ in
+ * tiling and scheduling, and several numbers may name one kernel). */
 int imresh_variant_counts(uint32_t width, uint32_t height, int *row_variants, int *col_variants);
 /* Pins the variants used for W x H on the current device instead of timing
  * them (a known tuning, or a test of one variant).  No reference
