@@ -130,16 +130,21 @@ int launch_variant(int mode, ColArgs a, hipStream_t s)
     const dim3 grid((a.W + C - 1) / C, images * (a.sub > 1 ? a.sub : 1)), block(C * P::T);
     constexpr size_t lds = col_lds<P, C>();
     constexpr int AJ = kAtJunction;
+    // the longest plans' projection pass is the four-step one
+    constexpr bool proj = BL || P::n < kFourStepMinLine;
     if constexpr (lds > 64 * 1024) {
         static const hipError_t attr = [&] {
             hipError_t e = hipSuccess;
             for (const void *f : {(const void *) k_col<P, C, CK_FWD, AJ, BL>,
                                   (const void *) k_col<P, C, CK_INV, AJ, BL>,
                                   (const void *) k_col<P, C, CK_FWD_REAL, AJ, BL>,
-                                  (const void *) k_col<P, C, CK_INV_REAL, AJ, BL>,
-                                  (const void *) k_col<P, C, CK_PROJ, WHEN, BL>})
+                                  (const void *) k_col<P, C, CK_INV_REAL, AJ, BL>})
                 if (e == hipSuccess)
                     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
+            if constexpr (proj)
+                if (e == hipSuccess)
+                    e = hipFuncSetAttribute((const void *) k_col<P, C, CK_PROJ, WHEN, BL>,
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
             return e;
         }();
         if (attr != hipSuccess) return from_hip(attr);
@@ -152,14 +157,18 @@ int launch_variant(int mode, ColArgs a, hipStream_t s)
         a.out = a.X;
         IMR_LAUNCH((k_col<P, C, CK_INV_REAL, AJ, BL>), grid, block, lds, s, a);
         break;
-    case COL_PROJ: IMR_LAUNCH((k_col<P, C, CK_PROJ, WHEN, BL>), grid, block, lds, s, a); break;
+    case COL_PROJ:
+        if constexpr (proj) IMR_LAUNCH((k_col<P, C, CK_PROJ, WHEN, BL>), grid, block, lds, s, a);
+        else return IMRESH_ERR_INVALID;
+        break;
     default: return IMRESH_ERR_INVALID;
     }
     return imr::launch_status(__FILE__, __LINE__);
 }
 
 // Column variants of a length: index = when * shapes + shape.  `when` is where
-// CK_PROJ reads the modulus (line_pair); shape 0 has the plan's tile, shape 1
+// CK_PROJ reads the modulus (line_pair; one choice where that pass is the
+// four-step one, whose middle step reads it at the junction); shape 0 has the plan's tile, shape 1
 // (1024 and 2048 points) 4-column tiles, twice the workgroups.
 template <int N, int... Rs>
 constexpr int col_shape_count()
@@ -168,7 +177,7 @@ constexpr int col_shape_count()
 }
 
 template <int N, int... Rs>
-constexpr int col_variant_count() { return 3 * col_shape_count<N, Rs...>(); }
+constexpr int col_variant_count() { return (N < kFourStepMinLine ? 3 : 1) * col_shape_count<N, Rs...>(); }
 
 // Bluestein kernels exist for the power-of-two convolution lengths, with half
 // as many columns per tile as the plan (measured fastest, see kBlueVariant)
@@ -178,8 +187,10 @@ constexpr bool blue_length() { return N >= 64 && N <= 2 * kMaxLine && (N & (N - 
 template <class P, int C>
 int launch_when(int when, int mode, ColArgs a, hipStream_t s)
 {
-    if (when == kEarly) return launch_variant<P, C, kEarly>(mode, a, s);
-    if (when == kAhead) return launch_variant<P, C, kAhead>(mode, a, s);
+    if constexpr (P::n < kFourStepMinLine) {
+        if (when == kEarly) return launch_variant<P, C, kEarly>(mode, a, s);
+        if (when == kAhead) return launch_variant<P, C, kAhead>(mode, a, s);
+    }
     return launch_variant<P, C>(mode, a, s);
 }
 

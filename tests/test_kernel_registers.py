@@ -46,3 +46,11 @@ def test_kernels_do_not_spill():
     assert sum("k_row" in k for k in kernels) > 100 and sum("k_col" in k for k in kernels) > 100
     over = {k: v for k, v in kernels.items() if v[0] > MAX_SPILLS or v[1] > MAX_SCRATCH}
     assert not over, over
+
+
+def test_four_step_columns_have_no_projection_kernel():
+    # columns of 8192 points project in the four-step pass, whose middle step
+    # is the 1024-point kernel: variants of their own would never be launched,
+    # yet timed against each other on the first call of a size
+    plain = [k for k in kernel_metadata(im.LIB_PATH) if re.search(r"k_col\w+PlanEILi16ELi8192E.*Lb0EEE", k)]
+    assert len(plain) == 4   # forward and inverse, complex and real input
