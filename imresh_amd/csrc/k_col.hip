@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(C *P::T, 4) k_col(ColArgs a)
         auto pre = [&](const auto &el) {
             el.load([&](int s, int o) { m[s] = M.get<float>(m0, 4u * (unsigned) o * (unsigned) MP); });
         };
-        auto mid = [&](auto &x, const auto &el) { modulus_project_line<P::E>(x, m, el); };
+        auto mid = [&](auto &x, const auto &el) { modulus_project_line<P::E>(x, m, el, valid); };
         auto sl = st(X);
         xpair<P, -1, +1, BL, WHEN>(v, tw, t, L, bl, g0, pre, mid, sl);
     }

@@ -42,7 +42,9 @@ __device__ __forceinline__ cf modulus_project(cf z, float m)
 // One test for all elements of the thread (of which any below the bound sends
 // the whole set through the per-element choice) keeps the common path free of
 // branches: a branch per element kept the reciprocal square roots of a
-// thread's elements from overlapping.
+// thread's elements from overlapping.  A thread that stores nothing (valid is
+// false: a column past the edge, all zeros) has no say in it, for it would send
+// its whole wave through the choice (column pass of 60x64: 5.8 us, 4.4 so).
 __device__ __forceinline__ cf modulus_project_fast(cf z, float n2, float m)
 {
     const float f = m * __builtin_amdgcn_rsqf(n2);
@@ -50,13 +52,14 @@ __device__ __forceinline__ cf modulus_project_fast(cf z, float n2, float m)
 }
 
 template <int E, class El>
-__device__ __forceinline__ void modulus_project_line(cf (&v)[E], const float (&m)[E], const El &el)
+__device__ __forceinline__ void modulus_project_line(cf (&v)[E], const float (&m)[E], const El &el, bool valid)
 {
     float low = 1e-30f;
     el.all([&](int s, int o) {
         const float n2 = v[s].x * v[s].x + v[s].y * v[s].y;
         if (el.inside(o)) low = fminf(low, n2);
     });
+    if (!valid) low = 1e-30f;
     if (low >= 1e-30f) {
         // (elements past the end of a line have modulus 0: they become 0 if
         // the reciprocal root stays finite)
