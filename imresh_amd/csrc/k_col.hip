@@ -28,9 +28,10 @@ enum ColKernel { CK_FWD, CK_INV, CK_PROJ, CK_FWD_REAL, CK_INV_REAL };
 
 // C columns per workgroup; WHEN (CK_PROJ only): where the measured modulus
 // is read (line_pair); BL: Bluestein kernels of column length a.len with P
-// the convolution plan.
+// the convolution plan.  At least 4 waves per SIMD; 3 for 32 points, whose 132
+// registers spill under the bound of 128 (64x32: 4.6 us, 4.1 so).
 template <class P, int C, int K, int WHEN = kAtJunction, bool BL = false>
-__global__ void __launch_bounds__(C *P::T, 4) k_col(ColArgs a)
+__global__ void __launch_bounds__(C *P::T, P::n == 32 ? 3 : 4) k_col(ColArgs a)
 {
     // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs
     // (workgroup x + y * gridDim.x to XCD (x + y * gridDim.x) mod 8), each

@@ -46,6 +46,8 @@ def test_kernels_do_not_spill():
     assert sum("k_row" in k for k in kernels) > 100 and sum("k_col" in k for k in kernels) > 100
     over = {k: v for k, v in kernels.items() if v[0] > MAX_SPILLS or v[1] > MAX_SCRATCH}
     assert not over, over
+    columns = {k: v for k, v in kernels.items() if "k_col" in k and v[0] > 0}
+    assert not columns, columns
 
 
 def test_four_step_columns_have_no_projection_kernel():
