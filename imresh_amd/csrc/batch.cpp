@@ -203,8 +203,7 @@ int work_stream(int device, hipStream_t *out)
 // pinned mirror, and the images' scalars and flags, cleared and read back by
 // one small kernel each.  Uploading, clearing and reading back class by class
 // with a synchronization each took 0.95 ms of a 24-image call.  Blocks above
-// kStageKeep, or that would take the idle buffers past the pool's cap, are
-// freed with the call.
+// kStageKeep are freed with the call.
 constexpr size_t kStageKeep = (size_t) 4 << 20;
 struct Stage {
     void *dev = nullptr;
@@ -257,28 +256,6 @@ Stage &stage_of(int device)
 {
     std::lock_guard<std::mutex> lk(g_mtx);
     return g_stage[device];
-}
-
-// f(block) for the block of every device that has no batch running
-template <class F>
-void idle_stages(F &&f)
-{
-    std::vector<int> devices;
-    {
-        std::lock_guard<std::mutex> lk(g_mtx);
-        for (auto &kv : g_stage) devices.push_back(kv.first);
-    }
-    for (int d : devices) {
-        std::unique_lock<std::mutex> run(run_lock(d), std::try_to_lock);
-        if (run.owns_lock()) f(stage_of(d));
-    }
-}
-
-// whether `bytes` more than the idle class buffers pass the pool's cap
-bool over_cap(size_t bytes)
-{
-    std::lock_guard<std::mutex> lk(g_mtx);
-    return g_idle + bytes > pool_cap();
 }
 
 struct Class {
@@ -497,7 +474,7 @@ int run_batch(const imresh_image *imgs, uint32_t count, const imresh_params *par
         if (kv.second.buf) class_return(kv.second.buf, s);
     if (exec) (void) hipGraphExecDestroy(exec);
     if (graph) (void) hipGraphDestroy(graph);
-    if (sg.bytes > kStageKeep || over_cap(sg.bytes)) sg.release();
+    if (sg.bytes > kStageKeep) sg.release();
     (void) hipEventDestroy(ev);
     return st;
 }
@@ -511,21 +488,25 @@ namespace imr {
 int trim_idle_classes(size_t cap)
 {
     std::vector<ClassBuf *> drop;
+    std::vector<int> devices;
     {
         std::lock_guard<std::mutex> lk(g_mtx);
         trim_classes(cap, drop);
+        if (cap == 0)
+            for (auto &kv : g_stage) devices.push_back(kv.first);
     }
     for (ClassBuf *x : drop) class_free(x);
-    idle_stages([](Stage &sg) { sg.release(); });
+    for (int d : devices) {   // the block of a device with no batch running
+        std::unique_lock<std::mutex> run(run_lock(d), std::try_to_lock);
+        if (run.owns_lock()) stage_of(d).release();
+    }
     return IMRESH_OK;
 }
 
 size_t idle_class_bytes()
 {
-    size_t bytes = 0;
-    idle_stages([&](Stage &sg) { bytes += sg.bytes; });
     std::lock_guard<std::mutex> lk(g_mtx);
-    return bytes + g_idle;
+    return g_idle;
 }
 
 }  // namespace imr

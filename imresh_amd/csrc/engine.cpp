@@ -1147,8 +1147,8 @@ int imresh_set_option(int option, int value)
             trim_idle(g_pool_cap, drop);
         }
         for (Workspace *x : drop) ws_release(x);
-        // the per-operator scratch, the reduction slots and the batches'
-        // per-call block are not kept under a new cap either
+        // the per-operator scratch and reduction slots are not kept under a
+        // new cap either
         reduce_slots_release();
         pool_bufs_release();
         return guarded([&] { return trim_idle_classes((size_t) value << 20); });
@@ -1179,10 +1179,8 @@ int imresh_cached_bytes(uint64_t *bytes)
         ws = g_idle_bytes;
     }
     // the pools' locks are never held together
-    return guarded([&] {
-        *bytes = ws + idle_class_bytes() + reduce_slots_bytes() + pool_bufs_bytes();
-        return (int) IMRESH_OK;
-    });
+    *bytes = ws + idle_class_bytes() + reduce_slots_bytes() + pool_bufs_bytes();
+    return IMRESH_OK;
 }
 
 int imresh_stream_create(void **stream)

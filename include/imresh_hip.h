@@ -95,19 +95,16 @@ int imresh_stream_sync(void *stream);
  * kernels one by one; both compute the same bits.  IMRESH_OPT_POOL_MIB: the
  * device memory (MiB, default 32768) that idle per-size workspaces may keep
  * between calls; beyond it the least recently used idle ones are freed
- * (setting it also frees the idle per-operator scratch and the per-call block
- * of the batches, which is not kept where it would pass the cap). */
+ * (setting it also frees the idle per-operator scratch). */
 enum { IMRESH_OPT_CYCLE_GRAPHS = 1, IMRESH_OPT_POOL_MIB = 2 };
 int imresh_set_option(int option, int value);
 /* Frees every idle pooled workspace and batch buffer whose work has
  * finished (all of them after the caller's streams are synchronized), the
- * per-call block of the batches, the idle scratch slots of the synchronous
- * reductions and the idle scratch buffers of the asynchronous per-operator
- * entry points. */
+ * idle scratch slots of the synchronous reductions and the idle scratch
+ * buffers of the asynchronous per-operator entry points. */
 int imresh_release_cached(void);
-/* Device bytes held by idle pooled workspaces, batch buffers, the batches'
- * per-call block (64 KiB to 4 MiB, and as much pinned host memory), reduction
- * scratch slots and per-operator scratch buffers. */
+/* Device bytes held by idle pooled workspaces, batch buffers and reduction
+ * scratch slots. */
 int imresh_cached_bytes(uint64_t *bytes);
 
 /* A non-blocking HIP stream at the default priority (for callers without a
