@@ -44,6 +44,9 @@ struct ClassBuf {
     uint8_t *mask = nullptr;
     float *pmax = nullptr, *perr = nullptr;
     unsigned *pcnt = nullptr;
+    float *scal = nullptr;   // [cap][kScalStride]
+    int *flags = nullptr;    // [cap][kFlagStride]
+    void **tab = nullptr;    // [cap] image pointers (gather / scatter)
     hipStream_t branch = nullptr;
     hipEvent_t join = nullptr, ready = nullptr;
     bool pending = false;
@@ -111,6 +114,9 @@ int class_alloc(int device, int W, int H, int cap, ClassBuf **out)
     const size_t oPmax = off; off = align256(off + 4 * ntiles);
     const size_t oPerr = off; off = align256(off + 4 * nrow);
     const size_t oPcnt = off; off = align256(off + 4 * nrow);
+    const size_t oScal = off; off = align256(off + sizeof(float) * kScalStride * cap);
+    const size_t oFlags = off; off = align256(off + sizeof(int) * kFlagStride * cap);
+    const size_t oTab = off; off = align256(off + sizeof(void *) * cap);
     c->bytes = off;
     hipError_t e = hipMalloc(&c->base, off);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->branch, hipStreamNonBlocking);
@@ -130,6 +136,9 @@ int class_alloc(int device, int W, int H, int cap, ClassBuf **out)
     c->pmax = (float *) (b + oPmax);
     c->perr = (float *) (b + oPerr);
     c->pcnt = (unsigned *) (b + oPcnt);
+    c->scal = (float *) (b + oScal);
+    c->flags = (int *) (b + oFlags);
+    c->tab = (void **) (b + oTab);
     *out = c;
     return IMRESH_OK;
 }
@@ -197,72 +206,8 @@ int work_stream(int device, hipStream_t *out)
     return IMRESH_OK;
 }
 
-// Per-call device block of a batch, kept per device between calls (one batch
-// runs on a device at a time, under its run lock, and ends synchronized):
-// inputs [weights rows][image pointers], uploaded by one copy from their
-// pinned mirror, and the images' scalars and flags, cleared and read back by
-// one small kernel each.  Uploading, clearing and reading back class by class
-// with a synchronization each took 0.95 ms of a 24-image call.  Blocks above
-// kStageKeep are freed with the call.
-constexpr size_t kStageKeep = (size_t) 4 << 20;
-struct Stage {
-    void *dev = nullptr;
-    char *host = nullptr;   // pinned: the inputs, then the results
-    size_t bytes = 0;
-    float *weights = nullptr, *scal = nullptr;
-    void **tab = nullptr;
-    int *flags = nullptr;
-    size_t in_bytes = 0, state_words = 0;
-
-    void release()
-    {
-        if (dev) (void) hipFree(dev);
-        if (host) (void) hipHostFree(host);
-        dev = nullptr;
-        host = nullptr;
-        bytes = 0;
-    }
-    int reserve(size_t weight_floats, size_t count)
-    {
-        const size_t oTab = align256(sizeof(float) * weight_floats);
-        in_bytes = align256(oTab + sizeof(void *) * count);
-        const size_t oFlags = align256(in_bytes + sizeof(float) * kScalStride * count);
-        const size_t need = align256(oFlags + sizeof(int) * kFlagStride * count);
-        if (need > bytes) {
-            release();
-            size_t cap = 1 << 16;
-            while (cap < need) cap <<= 1;
-            IMR_HIP_CHECK(hipMalloc(&dev, cap));
-            const hipError_t e = hipHostMalloc((void **) &host, cap, hipHostMallocCoherent);
-            if (e != hipSuccess) {
-                release();
-                return from_hip(e);
-            }
-            bytes = cap;
-        }
-        weights = (float *) dev;
-        tab = (void **) ((char *) dev + oTab);
-        scal = (float *) ((char *) dev + in_bytes);
-        flags = (int *) ((char *) dev + oFlags);
-        state_words = (need - in_bytes) / sizeof(float);
-        return IMRESH_OK;
-    }
-    template <class T>
-    T *mirror(T *d) const { return (T *) (host + ((char *) d - (char *) dev)); }
-};
-std::map<int, Stage> g_stage;   // by device, used under its run lock
-
-Stage &stage_of(int device)
-{
-    std::lock_guard<std::mutex> lk(g_mtx);
-    return g_stage[device];
-}
-
 struct Class {
     int W, H;
-    size_t first = 0;       // place of the class's images in the stage's arrays
-    float *scal = nullptr;  // [count][kScalStride]
-    int *flags = nullptr;   // [count][kFlagStride]
     std::vector<int> idx;   // positions in the caller's list
     ClassBuf *buf = nullptr;
     Plan2D p;
@@ -282,29 +227,29 @@ int enqueue_cycle(const Class &k, const Params &q, const float *weights, int R, 
     ba.W = k.W;
     ba.H = k.H;
     ba.pmax = c->pmax;
-    ba.done = k.flags;
+    ba.done = c->flags;
     ba.batch = B;
     ba.istride = c->n;
-    ba.cycles = (const unsigned *) (k.flags + 1);
+    ba.cycles = (const unsigned *) (c->flags + 1);
     IMR_CHECK(launch_blur(ba, s));
-    IMR_CHECK(launch_max_finalize_batch(c->pmax, k.ntiles, q.cutA, q.cut, k.scal, k.flags, B, s));
+    IMR_CHECK(launch_max_finalize_batch(c->pmax, k.ntiles, q.cutA, q.cut, c->scal, c->flags, B, s));
     RowArgs ra{};
     ra.X = c->X;
     ra.G = c->G;
     ra.mask = c->mask;
     ra.Bn = c->Bn;
     ra.B2 = c->B2;
-    ra.thr = k.scal;
+    ra.thr = c->scal;
     ra.beta = q.beta;
     ra.perr = c->perr;
     ra.pcnt = c->pcnt;
-    ra.done = k.flags;
+    ra.done = c->flags;
     ra.batch = B;
     ra.istride = c->n;
     ColArgs ca{};
     ca.X = c->X;
     ca.M = c->M;
-    ca.done = k.flags;
+    ca.done = c->flags;
     ca.batch = B;
     ca.istride = c->n;
     for (unsigned it = 0; it < q.n_hio; ++it) {
@@ -312,7 +257,7 @@ int enqueue_cycle(const Class &k, const Params &q, const float *weights, int R, 
         IMR_CHECK(launch_col(COL_PROJ, k.p, ca, s));
     }
     IMR_CHECK(launch_row(ROW_LAST, k.p, ra, s));
-    return launch_err_finalize_batch(c->perr, c->pcnt, k.nrowwg, q.target, k.scal, k.flags, B, s);
+    return launch_err_finalize_batch(c->perr, c->pcnt, k.nrowwg, q.target, c->scal, c->flags, B, s);
 }
 
 int run_batch(const imresh_image *imgs, uint32_t count, const imresh_params *params, hipStream_t user,
@@ -343,11 +288,9 @@ int run_batch(const imresh_image *imgs, uint32_t count, const imresh_params *par
     std::lock_guard<std::mutex> run(run_lock(dev));
     hipStream_t s;
     IMR_CHECK(work_stream(dev, &s));
-    Stage &sg = stage_of(dev);
-    IMR_CHECK(sg.reserve(wrows.size(), count));
-    float *const weights = sg.weights;
     hipEvent_t ev = nullptr;
     IMR_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    float *weights = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int st = IMRESH_OK;
@@ -358,80 +301,81 @@ int run_batch(const imresh_image *imgs, uint32_t count, const imresh_params *par
     // the work stream follows the caller's stream
     hip(hipEventRecord(ev, user));
     hip(hipStreamWaitEvent(s, ev, 0));
-    size_t placed = 0;
     for (auto &kv : classes) {
         Class &k = kv.second;
-        int rv, cv;
-        if (st == IMRESH_OK && !get_tuned_variants(dev, k.W, k.H, &rv, &cv)) st = tune_size(dev, k.W, k.H, s);
+        if (st == IMRESH_OK) st = tune_size(dev, k.W, k.H, s);
         if (st == IMRESH_OK) st = get_plan2d(dev, k.W, k.H, &k.p);
         if (st == IMRESH_OK) st = class_checkout(dev, k.W, k.H, (int) k.idx.size(), s, &k.buf);
         if (st != IMRESH_OK) break;
         k.nrowwg = row_grid(k.p);
         k.ntiles = blur_grid(k.W, k.H);
-        k.first = placed;
-        k.scal = sg.scal + kScalStride * placed;
-        k.flags = sg.flags + kFlagStride * placed;
-        for (int i : k.idx) sg.mirror(sg.tab)[placed++] = imgs[i].data;
     }
-    std::memcpy(sg.host, wrows.data(), sizeof(float) * wrows.size());
-    hip(hipMemcpyAsync(sg.dev, sg.host, sg.in_bytes, hipMemcpyHostToDevice, s));
-    if (st == IMRESH_OK) st = launch_zero_words(sg.scal, (unsigned) sg.state_words, s);
+    hip(hipMallocAsync((void **) &weights, sizeof(float) * wrows.size(), s));
+    hip(hipMemcpyAsync(weights, wrows.data(), sizeof(float) * wrows.size(), hipMemcpyHostToDevice, s));
 
-    // runs `work` for every class on its own branch stream, between what is
-    // queued on s before and after
-    auto on_branches = [&](auto work) {
-        hip(hipEventRecord(ev, s));
-        for (auto &kv : classes) {
-            Class &k = kv.second;
-            if (st != IMRESH_OK) break;
-            hip(hipStreamWaitEvent(k.buf->branch, ev, 0));
-            if (st == IMRESH_OK) st = work(k, k.buf->branch);
-            hip(hipEventRecord(k.buf->join, k.buf->branch));
-            hip(hipStreamWaitEvent(s, k.buf->join, 0));
+    // inputs, state reset and the initial inverse transform of every class
+    std::vector<void *> tab;
+    for (auto &kv : classes) {
+        if (st != IMRESH_OK) break;
+        Class &k = kv.second;
+        ClassBuf *c = k.buf;
+        const int B = (int) k.idx.size();
+        if (device_io) {
+            tab.assign(B, nullptr);
+            for (int b = 0; b < B; ++b) tab[b] = imgs[k.idx[b]].data;
+            hip(hipMemcpyAsync(c->tab, tab.data(), sizeof(void *) * B, hipMemcpyHostToDevice, s));
+            hip(hipStreamSynchronize(s));   // tab is reused for the next class
+            if (st == IMRESH_OK) st = launch_gather_images(c->M, (const float *const *) c->tab, c->n, B, s);
+        } else {
+            for (int b = 0; b < B; ++b)
+                hip(hipMemcpyAsync(c->M + (size_t) b * c->n, imgs[k.idx[b]].data, sizeof(float) * c->n,
+                                   hipMemcpyHostToDevice, s));
         }
-    };
-
-    // inputs and the initial inverse transform of every class
-    if (st == IMRESH_OK)
-        on_branches([&](Class &k, hipStream_t bs) {
-            ClassBuf *c = k.buf;
-            const int B = (int) k.idx.size();
-            if (device_io) {
-                IMR_CHECK(launch_gather_images(c->M, (const float *const *) (sg.tab + k.first), c->n, B, bs));
-            } else {
-                for (int b = 0; b < B; ++b)
-                    IMR_HIP_CHECK(hipMemcpyAsync(c->M + (size_t) b * c->n, imgs[k.idx[b]].data,
-                                                 sizeof(float) * c->n, hipMemcpyHostToDevice, bs));
-            }
-            ColArgs ca{};
-            ca.X = c->X;
-            ca.M = c->M;
-            ca.done = k.flags;
-            ca.batch = B;
-            ca.istride = c->n;
-            IMR_CHECK(launch_col(COL_INIT, k.p, ca, bs));
-            RowArgs ra{};
-            ra.X = c->X;
-            ra.G = c->G;
-            ra.mask = c->mask;
-            ra.Bn = c->Bn;
-            ra.done = k.flags;
-            ra.batch = B;
-            ra.istride = c->n;
-            return launch_row(ROW_INIT, k.p, ra, bs);
-        });
+        hip(hipMemsetAsync(c->scal, 0, sizeof(float) * kScalStride * B, s));
+        hip(hipMemsetAsync(c->flags, 0, sizeof(int) * kFlagStride * B, s));
+        ColArgs ca{};
+        ca.X = c->X;
+        ca.M = c->M;
+        ca.done = c->flags;
+        ca.batch = B;
+        ca.istride = c->n;
+        if (st == IMRESH_OK) st = launch_col(COL_INIT, k.p, ca, s);
+        RowArgs ra{};
+        ra.X = c->X;
+        ra.G = c->G;
+        ra.mask = c->mask;
+        ra.Bn = c->Bn;
+        ra.done = c->flags;
+        ra.batch = B;
+        ra.istride = c->n;
+        if (st == IMRESH_OK) st = launch_row(ROW_INIT, k.p, ra, s);
+    }
 
     // one cycle of every class as a graph, each class on its own branch;
     // without graphs every class runs all its cycles on its own stream
     if (st == IMRESH_OK && q.n_cycles > 0) st = prepare_blur(R);
     if (st == IMRESH_OK && q.n_cycles > 0 && !g_use_graphs) {
-        on_branches([&](Class &k, hipStream_t bs) {
-            for (unsigned cyc = 0; cyc < q.n_cycles; ++cyc) IMR_CHECK(enqueue_cycle(k, q, weights, R, bs));
-            return (int) IMRESH_OK;
-        });
+        hip(hipEventRecord(ev, s));
+        for (auto &kv : classes) {
+            Class &k = kv.second;
+            if (st != IMRESH_OK) break;
+            hip(hipStreamWaitEvent(k.buf->branch, ev, 0));
+            for (unsigned cyc = 0; cyc < q.n_cycles && st == IMRESH_OK; ++cyc)
+                st = enqueue_cycle(k, q, weights, R, k.buf->branch);
+            hip(hipEventRecord(k.buf->join, k.buf->branch));
+            hip(hipStreamWaitEvent(s, k.buf->join, 0));
+        }
     } else if (st == IMRESH_OK && q.n_cycles > 0) {
         hip(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-        on_branches([&](Class &k, hipStream_t bs) { return enqueue_cycle(k, q, weights, R, bs); });
+        hip(hipEventRecord(ev, s));
+        for (auto &kv : classes) {
+            Class &k = kv.second;
+            if (st != IMRESH_OK) break;
+            hip(hipStreamWaitEvent(k.buf->branch, ev, 0));
+            if (st == IMRESH_OK) st = enqueue_cycle(k, q, weights, R, k.buf->branch);
+            hip(hipEventRecord(k.buf->join, k.buf->branch));
+            hip(hipStreamWaitEvent(s, k.buf->join, 0));
+        }
         const hipError_t ec = hipStreamEndCapture(s, &graph);
         hip(ec);
         if (st == IMRESH_OK) hip(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
@@ -439,42 +383,49 @@ int run_batch(const imresh_image *imgs, uint32_t count, const imresh_params *par
     }
 
     // outputs Re(g') and the per-image results
-    if (st == IMRESH_OK)
-        on_branches([&](Class &k, hipStream_t bs) {
-            ClassBuf *c = k.buf;
-            const int B = (int) k.idx.size();
-            if (device_io) return launch_scatter_real((float *const *) (sg.tab + k.first), c->X, c->n, B, bs);
-            IMR_CHECK(launch_copy_from_real(c->B2, c->X, c->n * B, bs));
-            for (int b = 0; b < B; ++b)
-                IMR_HIP_CHECK(hipMemcpyAsync(imgs[k.idx[b]].data, c->B2 + (size_t) b * c->n,
-                                             sizeof(float) * c->n, hipMemcpyDeviceToHost, bs));
-            return (int) IMRESH_OK;
-        });
-    if (st == IMRESH_OK && results != nullptr)
-        st = launch_stage_words(sg.mirror(sg.scal), sg.scal, (unsigned) sg.state_words, s);
-    hipError_t es = hipStreamSynchronize(s);
-    hip(es);
-    if (st == IMRESH_OK && results != nullptr)
-        for (auto &kv : classes) {
-            const Class &k = kv.second;
-            const float *sc = sg.mirror(k.scal);
-            const int *fl = sg.mirror(k.flags);
-            for (size_t b = 0; b < k.idx.size(); ++b) {
-                imresh_result &r = results[k.idx[b]];
-                r.cycles_run = (uint32_t) fl[b * kFlagStride + 1];
-                r.last_error = sc[b * kScalStride + 1];
-                r.last_total = sc[b * kScalStride + 2];
-                r.last_masked = sc[b * kScalStride + 3];
+    std::vector<float> sc;
+    std::vector<int> fl;
+    for (auto &kv : classes) {
+        Class &k = kv.second;
+        ClassBuf *c = k.buf;
+        if (c == nullptr) continue;
+        const int B = (int) k.idx.size();
+        if (st == IMRESH_OK) {
+            if (device_io) {
+                tab.assign(B, nullptr);
+                for (int b = 0; b < B; ++b) tab[b] = imgs[k.idx[b]].data;
+                hip(hipMemcpyAsync(c->tab, tab.data(), sizeof(void *) * B, hipMemcpyHostToDevice, s));
+                hip(hipStreamSynchronize(s));
+                if (st == IMRESH_OK) st = launch_scatter_real((float *const *) c->tab, c->X, c->n, B, s);
+            } else {
+                if (st == IMRESH_OK) st = launch_copy_from_real(c->B2, c->X, c->n * B, s);
+                for (int b = 0; b < B; ++b)
+                    hip(hipMemcpyAsync(imgs[k.idx[b]].data, c->B2 + (size_t) b * c->n, sizeof(float) * c->n,
+                                       hipMemcpyDeviceToHost, s));
             }
         }
-    if (st != IMRESH_OK)   // whatever a failed call left on the branches
-        for (auto &kv : classes)
-            if (kv.second.buf) (void) hipStreamSynchronize(kv.second.buf->branch);
+        if (st == IMRESH_OK && results != nullptr) {
+            sc.assign((size_t) kScalStride * B, 0.f);
+            fl.assign((size_t) kFlagStride * B, 0);
+            hip(hipMemcpyAsync(sc.data(), c->scal, sizeof(float) * sc.size(), hipMemcpyDeviceToHost, s));
+            hip(hipMemcpyAsync(fl.data(), c->flags, sizeof(int) * fl.size(), hipMemcpyDeviceToHost, s));
+            hip(hipStreamSynchronize(s));
+            for (int b = 0; b < B && st == IMRESH_OK; ++b) {
+                imresh_result &r = results[k.idx[b]];
+                r.cycles_run = (uint32_t) fl[(size_t) b * kFlagStride + 1];
+                r.last_error = sc[(size_t) b * kScalStride + 1];
+                r.last_total = sc[(size_t) b * kScalStride + 2];
+                r.last_masked = sc[(size_t) b * kScalStride + 3];
+            }
+        }
+    }
+    hipError_t es = hipStreamSynchronize(s);
+    hip(es);
     for (auto &kv : classes)
         if (kv.second.buf) class_return(kv.second.buf, s);
     if (exec) (void) hipGraphExecDestroy(exec);
     if (graph) (void) hipGraphDestroy(graph);
-    if (sg.bytes > kStageKeep) sg.release();
+    if (weights) (void) hipFreeAsync(weights, s);
     (void) hipEventDestroy(ev);
     return st;
 }
@@ -488,18 +439,11 @@ namespace imr {
 int trim_idle_classes(size_t cap)
 {
     std::vector<ClassBuf *> drop;
-    std::vector<int> devices;
     {
         std::lock_guard<std::mutex> lk(g_mtx);
         trim_classes(cap, drop);
-        if (cap == 0)
-            for (auto &kv : g_stage) devices.push_back(kv.first);
     }
     for (ClassBuf *x : drop) class_free(x);
-    for (int d : devices) {   // the block of a device with no batch running
-        std::unique_lock<std::mutex> run(run_lock(d), std::try_to_lock);
-        if (run.owns_lock()) stage_of(d).release();
-    }
     return IMRESH_OK;
 }
 
