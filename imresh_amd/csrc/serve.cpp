@@ -422,13 +422,15 @@ static int server_submit_impl(imresh_server *h, float *io, uint32_t width, uint3
         return IMRESH_ERR_BUDGET;
     }
     r->t_submit = imr::Clock::now();
+    uint64_t given;
     {
         std::lock_guard<std::mutex> lk(s.mtx);
-        r->id = s.next_id++;
+        given = r->id = s.next_id++;
         ++s.submitted;
         s.queue.push_back(r);
     }
-    if (id) *id = r->id;
+    // (the request may be complete and gone by now)
+    if (id) *id = given;
     s.cv.notify_one();
     return IMRESH_OK;
 }
