@@ -87,9 +87,10 @@ void trim_classes(size_t cap, std::vector<ClassBuf *> &out)
 void class_free(ClassBuf *c)
 {
     if (c->base) (void) hipFree(c->base);
-    if (c->branch) (void) hipStreamDestroy(c->branch);
+    // the events first: one recorded on a stream does not outlive it
     if (c->join) (void) hipEventDestroy(c->join);
     if (c->ready) (void) hipEventDestroy(c->ready);
+    if (c->branch) (void) hipStreamDestroy(c->branch);
     delete c;
 }
 

@@ -190,6 +190,33 @@ int launch_scatter_real(float *const *, const float2 *, size_t, int, hipStream_t
 int launch_copy_from_real(float *, const float2 *, size_t, hipStream_t) { return IMRESH_OK; }
 }  // namespace imr
 
+static void batches()
+{
+    imresh_params p{};
+    p.n_cycles = 2;
+    p.n_hio_cycles = 1;
+    for (int graphs = 0; graphs < 2; ++graphs) {
+        imr::g_use_graphs = graphs != 0;
+        for (int host = 0; host < 2; ++host) {
+            std::vector<std::vector<float>> mem;
+            std::vector<imresh_image> im;
+            for (uint32_t n : {4u, 6u, 4u, 8u, 5u}) {
+                mem.emplace_back((size_t) n * n, 1.f);
+                im.push_back({mem.back().data(), n, n});
+            }
+            std::vector<imresh_result> res(im.size());
+            for (int rep = 0; rep < 3; ++rep) {
+                const int st = host ? imresh_shrinkwrap_batch(im.data(), (uint32_t) im.size(), &p, nullptr, res.data())
+                                    : imresh_shrinkwrap_batch_device(im.data(), (uint32_t) im.size(), &p, nullptr,
+                                                                     rep ? res.data() : nullptr);
+                expect(st == IMRESH_OK, "batch status");
+            }
+        }
+        imr::trim_idle_classes(0);
+    }
+    expect(imr::idle_class_bytes() == 0, "idle bytes after the release");
+}
+
 static void requests()
 {
     imresh_params p{};
@@ -208,6 +235,7 @@ static void requests()
 
 int main()
 {
+    batches();
     requests();
     std::printf("%d lifetime errors\n", g_bad);
     return g_bad != 0;
