@@ -75,8 +75,9 @@ __device__ __forceinline__ void blue_apply_chirp(cf (&v)[PM::E], const Chirp<PM>
 // circular convolution with the chirp: v holds the chirped line (zero from n
 // to M/2; the zeros of the upper half are implied, their registers not read)
 // at PM's forward first-pass input positions on entry and the result at PM's
-// inverse last-pass output positions on exit.  The chirp's spectrum is loaded after the forward transform's last pass; `hook` runs after the
-// inverse's (loads issued before the last exchange take registers from its
+// inverse last-pass output positions on exit.  The chirp's spectrum is loaded
+// after the forward transform's last pass; `hook` runs after the inverse's
+// (loads issued before the last exchange take registers from its
 // butterflies: 1373 x 1101, 10 iterations 793 us so, 923 us with them ahead).
 template <class PM, int DIR, class Lds, class Hook>
 __device__ __forceinline__ void blue_conv(cf (&v)[PM::E], const Buf &tw, int t, const Lds &L,

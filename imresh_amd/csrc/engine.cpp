@@ -227,8 +227,8 @@ int ws_checkout(int device, int W, int H, hipStream_t s, Workspace **out)
     // a busy workspace taken over (kMaxWorkspaces of this size in use): its
     // previous user's work runs first.  Should that work not finish in
     // reasonable time (a caller stream destroyed with its work dropped would
-    // never run the kernel that marks it idle), the workspace stays in the pool and a
-    // new one is allocated instead of waiting on.
+    // never run the kernel that marks it idle), the workspace stays in the
+    // pool and a new one is allocated instead of waiting on.
     (void) s;
     if (!ws_wait_idle(w, 10.0)) {
         {

@@ -44,7 +44,8 @@ struct Workspace {
     std::vector<float> host_weights;   // host copy of the weights table
     float *host_wpin = nullptr;        // pinned staging of that table (the upload's source)
     size_t host_wpin_n = 0;            // its capacity in floats
-    float *host_stage = nullptr;  // pinned, 64 floats + readback
+    // pinned, 4 KiB: the staged scalars and flags, done_word at byte 2048
+    float *host_stage = nullptr;
     // set when a user returns the workspace with work still queued on its
     // stream; the work has run once done_word (pinned, stored by a kernel
     // queued behind it) holds done_seq.  (An event recorded on the user's

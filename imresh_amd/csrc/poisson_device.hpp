@@ -97,9 +97,10 @@ __host__ __device__ inline double sqrt_d(double x)
 }
 
 // (float) sqrt_d(k) of an integer-valued k >= 0.  Below 2^24 the correctly
-// rounded single-precision root is the same: k is exact in float, and
-// sqrt(k) is never within 2^-50 (relative) of the midpoint of two floats,
-// whose square would differ from k by less than its last bit.
+// rounded single-precision root is the same: k is exact in float, and the
+// square of a midpoint m of two floats, an odd multiple of 2^(2e-48) for m in
+// [2^e, 2^(e+1)), differs from k by at least that, so sqrt(k) keeps a relative
+// distance of 2^-51 from m, more than twice the error of sqrt_d (below 2^-52).
 __host__ __device__ inline float sqrt_count(double k)
 {
     return k < 16777216.0 ? sqrtf((float) k) : (float) sqrt_d(k);
@@ -130,7 +131,8 @@ struct Reciprocals {
 };
 
 // x / k, correctly rounded as the division is, for 1 <= k <= kCount and x >= 0
-// far from underflow: x*hi + x*lo is exact to 2^-104, a quotient by k keeps
+// far from underflow (the sampler's steps that underflow no longer change its
+// sum): x*hi + x*lo is exact to 2^-104, a quotient by k keeps
 // 2^-60 from every rounding boundary and is never on one (k times an odd
 // 54-bit number has more than 53 bits).
 __host__ __device__ inline double div_small(double x, int k, const Reciprocals &r)
