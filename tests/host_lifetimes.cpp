@@ -4,7 +4,7 @@
 //   - an event is used and destroyed before the stream it was last recorded
 //     on (the runtime reads that stream);
 //   - a request that completes at once is not read by the call that
-//     submitted it (the thread checker sees it).
+//     submitted it (the thread sanitizer sees it).
 #include <cstdio>
 #include <cstdlib>
 #include <set>

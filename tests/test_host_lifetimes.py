@@ -1,6 +1,6 @@
 """Lifetimes of streams, events and requests in the server and the batch,
 checked on the host against a stand-in runtime (host_lifetimes.cpp), the
-server's threads under the thread checker."""
+server's threads under the thread sanitizer."""
 import os
 import subprocess
 
